@@ -471,7 +471,9 @@ struct theseus_rhs {
   float *d_lte32 = nullptr;   // mixed precision: the planes in FP32
   double *d_lteT = nullptr;   // per node: recovered temperature of the stage state
   int *d_ltecell = nullptr;   // per node: its table cell
-  double *d_ltepcg = nullptr; // per node, pairs other than LTEEC: pressure, sound speed (, gamma)
+  double *d_ltepcg = nullptr; // per node: pressure, sound speed (, gamma); LTEEC: sound speed (, pressure)
+  void *d_lterec = nullptr;   // LTEEC, per node: H and its derivatives
+  void *d_ltecells = nullptr; // LTEEC: the table's cell records
   BasisArgs basis;
   GasC<double> gas;
   GasC<float> gas32;
@@ -911,6 +913,35 @@ static int create_impl(const theseus_case_desc *desc, const theseus_lte_table *l
       }
       h->ltev.planes32 = h->d_lte32;
     }
+    if (lfx == LTE_FLUX_LTEEC) {
+      // node arrays (sound speed, and in the mixed form pressure, in FP64; H
+      // and its derivatives in the pair fluxes' type) and the cell records
+      const size_t rsz = h->pm ? sizeof(float) : sizeof(double);
+      char *rec = nullptr, *cells = nullptr;
+      if ((rc = upload<double>(&h->d_ltepcg, nullptr, (h->pm ? 2 : 1) * (size_t)h->Ntot)) ||
+          (rc = upload<char>(&rec, nullptr, 5 * rsz * h->Ntot)) ||
+          (rc = upload<char>(&cells, nullptr, lte::kCellStride * rsz * nx * ny))) {
+        hipFree(rec);
+        theseus_rhs_destroy(h);
+        return rc;
+      }
+      h->d_lterec = rec;
+      h->d_ltecells = cells;
+      h->ltev.node_c = h->d_ltepcg;
+      h->ltev.node_p = h->pm ? h->d_ltepcg + h->Ntot : nullptr;
+      h->ltev.node_rec = rec;
+      h->ltev.rec32 = h->pm;
+      const dim3 grid((unsigned)((nx * ny + 255) / 256));
+      if (h->pm) hipLaunchKernelGGL(lte::k_lte_cells<float>, grid, dim3(256), 0, nullptr, h->ltev, (float *)cells);
+      else hipLaunchKernelGGL(lte::k_lte_cells<double>, grid, dim3(256), 0, nullptr, h->ltev, (double *)cells);
+      hipError_t le = hipGetLastError();
+      if (le == hipSuccess) le = hipStreamSynchronize(nullptr);
+      if (le != hipSuccess) {
+        theseus_rhs_destroy(h);
+        return fail(THESEUS_ERR_DEVICE, std::string("LTE cell records: ") + hipGetErrorString(le));
+      }
+      h->ltev.cells = cells;
+    }
   }
   if (d.elem_orient) {
     const std::vector<Sym> syms = symmetries(dim);
@@ -1005,6 +1036,8 @@ int theseus_rhs_destroy(theseus_rhs *h) {
   hipFree(h->d_lteT);
   hipFree(h->d_ltecell);
   hipFree(h->d_ltepcg);
+  hipFree(h->d_lterec);
+  hipFree(h->d_ltecells);
   hipFree(h->d_stage[0]);
   hipFree(h->d_stage[1]);
   hipFree(h->d_rates);
@@ -1092,7 +1125,10 @@ static void enqueue_stability(theseus_rhs *h, const double *u, hipStream_t s) {
   if (h->lk) {
     // the tabulated gas: each node's temperature and cell recovered once
     // (k_lte_nodes), instead of a Newton solve per node and per face point
-    h->lk->nodes(h->args(u, nullptr), 0, s);
+    RHSArgs na = h->args(u, nullptr);
+    na.lte.node_p = nullptr;  // the recovery alone, not the fluxes' node values
+    na.lte.node_rec = nullptr;
+    h->lk->nodes(na, 0, s);
     a.lte_nodes = 1;
   }
   h->sk->stability(a, h->nblocks(), s);

@@ -40,6 +40,14 @@ struct View {
   // the Pirozzoli, HLL and LLF pairs: each node's pressure and sound speed
   // (and, for Pirozzoli, gamma = cp/cv), evaluated by k_lte_nodes; null for LTEEC
   double *node_p = nullptr, *node_c = nullptr, *node_g = nullptr;
+  // LTEEC: the scaled Hermite coefficients of every cell (kCellStride values
+  // of the arithmetic type per cell, k_lte_cells) and, per node, H, H_rho,
+  // H_rhorho, H_T and H_rhoT at its recovered temperature ([5][Ntot] of the
+  // arithmetic type, k_lte_node_rec, which writes node_c too and, in the
+  // mixed form, node_p); null for the other pairs
+  const void *cells = nullptr;
+  void *node_rec = nullptr;
+  int rec32 = 0;  // the records' arithmetic type: 0 FP64, 1 FP32
   // viscosity of the Navier-Stokes form: the mu plane, or Sutherland's law
   // mu0 (T0 + Ts) (T/T0)^1.5 / (T + Ts) when sutherland is set
   int sutherland = 0;
@@ -258,50 +266,111 @@ __device__ __forceinline__ double temperature_from_energy(const View &v, double 
   return __builtin_nan("");
 }
 
-enum class Q { pressure, gibbs };
-template <Q P, typename R>
-__device__ __forceinline__ R value(const Eval<R> &s) {
-  if constexpr (P == Q::pressure) return s.pressure();
-  else return s.gibbs();
+// ---- LTEEC: entropy-conserving means from per-node values and cell records
+
+// One cell's record (index j*nx + i): the 16 Hermite coefficients in
+// evaluate()'s order -- per corner (rho side, then T side) H, H_rho wr,
+// H_T wt, (H_rhoT wr) wt -- then wr, wt and the reciprocals of wr, wt, wr wr
+// and wr wt; two values of padding keep records on 64-byte lines.  A pair
+// reads one or two records of consecutive values instead of 32 values strided
+// over four planes and four grid points, with the scalings already applied.
+constexpr int kCellStride = 24;
+
+template <typename R>
+__global__ void __launch_bounds__(256) k_lte_cells(View v, R *out) {
+  const int t = blockIdx.x * blockDim.x + threadIdx.x;
+  const int i = t % v.nx, j = t / v.nx;
+  if (i >= v.nx - 1 || j >= v.ny - 1) return;
+  const Eval<R> ev = at_cell<R>(v, R(v.rho[i]), R(v.T[j]), i, j);
+  const Cell<R> &c = ev.cell;
+  R *o = out + (size_t)t * kCellStride;
+#pragma unroll
+  for (int ds = 0; ds < 2; ++ds)
+#pragma unroll
+    for (int ts = 0; ts < 2; ++ts) {
+      const int k = ds + ts * c.stride, m = 4 * (2 * ds + ts);
+      o[m] = c.H[k];
+      o[m + 1] = c.H[c.plane + k] * c.wr;
+      o[m + 2] = c.H[2 * c.plane + k] * c.wt;
+      o[m + 3] = c.H[3 * c.plane + k] * c.wr * c.wt;
+    }
+  o[16] = c.wr;
+  o[17] = c.wt;
+  o[18] = R(1) / c.wr;
+  o[19] = R(1) / c.wt;
+  o[20] = R(1) / (c.wr * c.wr);
+  o[21] = R(1) / (c.wr * c.wt);
 }
-template <Q P, typename R>
-__device__ __forceinline__ R density_secant(const Eval<R> &a, const Eval<R> &b, R eta) {
-  const Cell<R> &c = a.cell;
-  const R r1 = a.rho, r2 = b.rho;
-  const R h1 = evaluate<1, 0>(c, a.xi, eta);
-  const R h2 = evaluate<1, 0>(c, b.xi, eta);
-  const R mean_hr = R(0.5) * (h1 + h2);
-  const R div_hr = divided<0, 1, 0>(c, a.xi, eta, b.xi, eta);
-  if constexpr (P == Q::pressure) {
-    return R(0.5) * (r1 * r1 + r2 * r2) * div_hr + (r1 + r2) * mean_hr;
+
+// n / d with y the correctly rounded 1 / d: in FP64 the quotient estimate
+// n y corrected by its exact remainder, which rounds to the IEEE quotient in
+// three instructions instead of a division's eleven; FP32 divides.
+template <typename R>
+__device__ __forceinline__ R div_by(R n, R d, R y) {
+  if constexpr (sizeof(R) == sizeof(double)) {
+    const R q = n * y;
+    return fma(fma(-d, q, n), y, q);
   } else {
-    const R div_h = divided<0>(c, a.xi, eta, b.xi, eta);
-    return div_h + R(0.5) * (r1 + r2) * div_hr + mean_hr;
+    return n / d;
   }
 }
-template <Q P, typename R>
-__device__ __forceinline__ R beta_secant(const Eval<R> &a, const Eval<R> &b, R xi, R rho) {
-  const Cell<R> &c = a.cell;
-  const R mean_t = R(0.5) * (a.T + b.T);
-  const R h1 = evaluate<1, 0>(c, xi, a.eta);
-  const R h2 = evaluate<1, 0>(c, xi, b.eta);
-  const R mean_hr = R(0.5) * (h1 + h2);
-  const R div_hr = divided<1, 1, 0>(c, xi, a.eta, xi, b.eta);
-  const R hr_beta = mean_hr - mean_t * div_hr;
-  if constexpr (P == Q::pressure) {
-    return rho * rho * hr_beta;
-  } else {
-    const R g1 = evaluate<0, 0>(c, xi, a.eta);
-    const R g2 = evaluate<0, 0>(c, xi, b.eta);
-    const R mean_h = R(0.5) * (g1 + g2);
-    const R div_h = divided<1>(c, xi, a.eta, xi, b.eta);
-    return mean_h - mean_t * div_h + rho * hr_beta;
-  }
+
+// One node as an endpoint of a pair: H and H_rho at (rho, T), the cell (i | j
+// << 16) and the coordinates in it, beta = 1/T
+template <typename R>
+struct PairNode {
+  R rho, T, beta, xi, eta, H, Hr;
+  int cell;
+};
+
+// A node's endpoint from its state, recovered temperature and cell (-1:
+// outside the table, which makes every result NaN) and stored H, H_rho
+template <typename R>
+__device__ __forceinline__ PairNode<R> pair_node(const View &v, R rho, R T, int cell, R H, R Hr) {
+  const Eval<R> ev = at_packed<R>(v, rho, T, cell);
+  return PairNode<R>{rho, T, 1 / T, ev.xi, ev.eta, H, Hr, ev.ci | (ev.cj << 16)};
+}
+
+// Eval::pressure() of an endpoint
+template <typename R>
+__device__ __forceinline__ R pair_pressure(const PairNode<R> &s) {
+  return s.rho * s.rho * s.Hr;
+}
+
+// Products of a cell's coefficients with one rho basis (value side 0, 1,
+// slope side 0, 1), and their sum with one T basis: together evaluate()'s or
+// divided()'s operations in their order, the products shared by the T bases.
+template <typename R>
+struct Basis4 {
+  R v0, v1, s0, s1;
+};
+template <typename R>
+__device__ __forceinline__ void cell_row(const R *c, const Basis4<R> &b, R *P) {
+#pragma unroll
+  for (int m = 0; m < 16; ++m) P[m] = c[m] * (m < 8 ? ((m & 1) ? b.s0 : b.v0) : ((m & 1) ? b.s1 : b.v1));
 }
 template <typename R>
-struct Gradient {
-  R density = 0, beta = 0;
-};
+__device__ __forceinline__ R cell_dot(const R *P, const Basis4<R> &t) {
+  R r = 0;
+#pragma unroll
+  for (int m = 0; m < 16; ++m) r += P[m] * ((m & 4) ? ((m & 2) ? t.s1 : t.v1) : ((m & 2) ? t.s0 : t.v0));
+  return r;
+}
+// Keeps a value's computation where it is written: sunk into the branch that
+// uses it, a sum would drag its 16 products' registers along.
+template <typename R>
+__device__ __forceinline__ void pin(R &x) {
+  asm volatile("" : "+v"(x));
+}
+template <int D, typename R>
+__device__ __forceinline__ Basis4<R> basis4(R x) {
+  return Basis4<R>{pbasis<D>(0, x), pbasis<D>(1, x), sbasis<D>(0, x), sbasis<D>(1, x)};
+}
+template <int D, typename R>
+__device__ __forceinline__ Basis4<R> dbasis4(R x, R y) {
+  return Basis4<R>{dpbasis<D>(0, x, y), dpbasis<D>(1, x, y), dsbasis<D>(0, x, y), dsbasis<D>(1, x, y)};
+}
+
 // Below these differences the discrete gradient takes the derivative form
 // (LTEHelmholtzEOS.hpp:246-300): the reference's 2.22e-15 + 1.49e-8 x (about
 // 10 eps and sqrt(eps) of FP64), and the same multiples of FP32's epsilon
@@ -314,93 +383,140 @@ template <>
 struct SecantTol<float> {
   static constexpr float abs = 1.19e-6f, rel = 3.45e-4f;
 };
-template <Q P, typename R>
-__device__ __forceinline__ Gradient<R> discrete_gradient(const View &v, const Eval<R> &left, const Eval<R> &right) {
-  const bool reverse = left.rho > right.rho || (left.rho == right.rho && left.T > right.T);
-  const Eval<R> &a = reverse ? right : left;
-  const Eval<R> &b = reverse ? left : right;
-  const R b1 = 1 / a.T, b2 = 1 / b.T;
+
+// The order in which a pair enters the discrete gradients
+// (LTEHelmholtzEOS.hpp:231-244): by density, then temperature
+template <typename R>
+__device__ __forceinline__ bool pair_reversed(R rho1, R T1, R rho2, R T2) {
+  return rho1 > rho2 || (rho1 == rho2 && T1 > T2);
+}
+
+// The entropy-conserving density and energy means (LTEHelmholtzEOS.hpp:
+// 225-397) of an ordered pair: the Itoh-Abe discrete gradients of p/T and g/T
+// in (rho, 1/T).  `fall(side, k)` gives H_rhorho (2), H_T (3) or H_rhoT (4)
+// of endpoint a (0) or b (1) for the derivative form, rarely needed.
+//
+// Every evaluation at an endpoint itself comes with the nodes (evaluated
+// once per node and stage instead of in each of its pairs).  What is left is
+// H and H_rho at the two cross corners (rho_a, T_b) and (rho_b, T_a), needed
+// in both cases -- by the secants when the endpoints share a cell, by the
+// corner differences when not, the searches of at() then finding exactly the
+// cells (i_a, j_b) and (i_b, j_a) -- and, in a shared cell, eight divided
+// differences: 12 sums of 16 products from 6 rho bases, where taking each
+// gradient by itself evaluated 24 sums and 4 to 12 more per divergent branch.
+template <typename R, typename F>
+__device__ __forceinline__ void thermodynamic_means(const View &v, const PairNode<R> &a, const PairNode<R> &b, F fall,
+                                                    R &rho_mean, R &e_mean) {
+  const R b1 = a.beta, b2 = b.beta;
   const R dr = b.rho - a.rho, db = b2 - b1;
   const R rmax = a.rho > b.rho ? a.rho : b.rho;
   const R bmax = b1 > b2 ? b1 : b2;
   const bool dd = fabs(dr) >= R(SecantTol<R>::abs) + R(SecantTol<R>::rel) * rmax;
   const bool bd = fabs(db) >= R(SecantTol<R>::abs) + R(SecantTol<R>::rel) * bmax;
-  const R f11 = value<P>(a), f22 = value<P>(b);
-  Gradient<R> g;
-  const bool same_cell = a.cell.H == b.cell.H;
-  if (same_cell) {
-    if (dd) {
-      const R s1 = density_secant<P>(a, b, a.eta);
-      const R s2 = density_secant<P>(a, b, b.eta);
-      g.density = R(0.5) * (s1 * b1 + s2 * b2);
+  const R p11 = pair_pressure(a), p22 = pair_pressure(b);
+  const R g11 = a.H + a.rho * a.Hr, g22 = b.H + b.rho * b.Hr;
+  R pd = 0, gd = 0, pb = 0, gb = 0;  // the density and beta components of the two gradients
+  if (dd || bd) {
+    const int ia = a.cell & 0xFFFF, ja = a.cell >> 16, ib = b.cell & 0xFFFF, jb = b.cell >> 16;
+    const bool same = a.cell == b.cell;
+    const R *ca = static_cast<const R *>(v.cells) + (size_t)(jb * v.nx + ia) * kCellStride;
+    const R *cb = static_cast<const R *>(v.cells) + (size_t)(ja * v.nx + ib) * kCellStride;
+    const Basis4<R> dt = dbasis4<0, R>(a.eta, b.eta);
+    R c[16], P[16];
+    R hx, gx, hdt_a, gdt_a, hy, gy, hdt_b, gdt_b;
+    {
+      const Basis4<R> tb = basis4<0, R>(b.eta);
+#pragma unroll
+      for (int m = 0; m < 16; ++m) c[m] = ca[m];
+      cell_row(c, basis4<1, R>(a.xi), P);
+      hx = div_by(cell_dot(P, tb), ca[16], ca[18]);  // H_rho(rho_a, T_b)
+      hdt_a = cell_dot(P, dt);
+      pin(hdt_a);
+      __builtin_amdgcn_sched_barrier(0);
+      cell_row(c, basis4<0, R>(a.xi), P);
+      gx = cell_dot(P, tb);  // H(rho_a, T_b)
+      gdt_a = cell_dot(P, dt);
+      pin(gdt_a);
     }
-    if (bd) {
-      const R s1 = beta_secant<P>(a, b, a.xi, a.rho);
-      const R s2 = beta_secant<P>(a, b, b.xi, b.rho);
-      g.beta = R(0.5) * (s1 + s2);
+    {
+      __builtin_amdgcn_sched_barrier(0);
+      const Basis4<R> ta = basis4<0, R>(a.eta);
+#pragma unroll
+      for (int m = 0; m < 16; ++m) c[m] = cb[m];
+      cell_row(c, basis4<1, R>(b.xi), P);
+      hy = div_by(cell_dot(P, ta), cb[16], cb[18]);  // H_rho(rho_b, T_a)
+      hdt_b = cell_dot(P, dt);
+      pin(hdt_b);
+      __builtin_amdgcn_sched_barrier(0);
+      cell_row(c, basis4<0, R>(b.xi), P);
+      gy = cell_dot(P, ta);  // H(rho_b, T_a)
+      gdt_b = cell_dot(P, dt);
+      pin(gdt_b);
     }
-  } else if (dd || bd) {
-    // the cross corners (rho_a, T_b), (rho_b, T_a) lie in the cells (i_a, j_b)
-    // and (i_b, j_a): the searches of at() would find exactly these
-    const bool ok = a.valid && b.valid;
-    const R f12 = value<P>(ok ? at_cell<R>(v, a.rho, b.T, a.ci, b.cj) : at<R>(v, a.rho, b.T));
-    const R f21 = value<P>(ok ? at_cell<R>(v, b.rho, a.T, b.ci, a.cj) : at<R>(v, b.rho, a.T));
-    if (dd) g.density = R(0.5) * ((f21 * b1 - f11 * b1) + (f22 * b2 - f12 * b2)) / dr;
-    if (bd) g.beta = R(0.5) * ((f12 * b2 - f11 * b1) + (f22 * b2 - f21 * b1)) / db;
+    if (same) {
+      const R wr = cb[16], wt = cb[17], iwr = cb[18], iwt = cb[19], iwrr = cb[20], iwrt = cb[21];
+      if (dd) {
+        const Basis4<R> ta = basis4<0, R>(a.eta), tb = basis4<0, R>(b.eta);
+        cell_row(c, dbasis4<1, R>(a.xi, b.xi), P);
+        R dhr1 = div_by(cell_dot(P, ta), wr * wr, iwrr), dhr2 = div_by(cell_dot(P, tb), wr * wr, iwrr);
+        pin(dhr1);
+        pin(dhr2);
+        __builtin_amdgcn_sched_barrier(0);
+        cell_row(c, dbasis4<0, R>(a.xi, b.xi), P);
+        const R dh1 = div_by(cell_dot(P, ta), wr, iwr), dh2 = div_by(cell_dot(P, tb), wr, iwr);
+        const R m1 = R(0.5) * (a.Hr + hy), m2 = R(0.5) * (hx + b.Hr);
+        const R r2m = R(0.5) * (a.rho * a.rho + b.rho * b.rho), rs = a.rho + b.rho;
+        const R p1 = r2m * dhr1 + rs * m1, p2 = r2m * dhr2 + rs * m2;
+        pd = R(0.5) * (p1 * b1 + p2 * b2);
+        const R g1 = dh1 + R(0.5) * rs * dhr1 + m1, g2 = dh2 + R(0.5) * rs * dhr2 + m2;
+        gd = R(0.5) * (g1 * b1 + g2 * b2);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      if (bd) {
+        const R mean_t = R(0.5) * (a.T + b.T);
+        const R hb1 = R(0.5) * (a.Hr + hx) - mean_t * div_by(hdt_a, wr * wt, iwrt);
+        const R hb2 = R(0.5) * (hy + b.Hr) - mean_t * div_by(hdt_b, wr * wt, iwrt);
+        pb = R(0.5) * (a.rho * a.rho * hb1 + b.rho * b.rho * hb2);
+        const R g1 = R(0.5) * (a.H + gx) - mean_t * div_by(gdt_a, wt, iwt) + a.rho * hb1;
+        const R g2 = R(0.5) * (gy + b.H) - mean_t * div_by(gdt_b, wt, iwt) + b.rho * hb2;
+        gb = R(0.5) * (g1 + g2);
+      }
+    } else {
+      const R p12 = a.rho * a.rho * hx, p21 = b.rho * b.rho * hy;
+      const R g12 = gx + a.rho * hx, g21 = gy + b.rho * hy;
+      if (dd) {
+        const R y = 1 / dr;
+        pd = div_by(R(0.5) * ((p21 * b1 - p11 * b1) + (p22 * b2 - p12 * b2)), dr, y);
+        gd = div_by(R(0.5) * ((g21 * b1 - g11 * b1) + (g22 * b2 - g12 * b2)), dr, y);
+      }
+      if (bd) {
+        const R y = 1 / db;
+        pb = div_by(R(0.5) * ((p12 * b2 - p11 * b1) + (p22 * b2 - p21 * b1)), db, y);
+        gb = div_by(R(0.5) * ((g12 * b2 - g11 * b1) + (g22 * b2 - g21 * b1)), db, y);
+      }
+    }
   }
   if (!dd) {
-    if constexpr (P == Q::pressure) g.density = R(0.5) * (a.p_rho() * b1 + b.p_rho() * b2);
-    else g.density = R(0.5) * (a.g_rho() * b1 + b.g_rho() * b2);
+    const R h1 = fall(0, 2), h2 = fall(1, 2);  // H_rhorho
+    pd = R(0.5) * ((2 * a.rho * a.Hr + a.rho * a.rho * h1) * b1 + (2 * b.rho * b.Hr + b.rho * b.rho * h2) * b2);
+    gd = R(0.5) * ((2 * a.Hr + a.rho * h1) * b1 + (2 * b.Hr + b.rho * h2) * b2);
   }
   if (!bd) {
-    R d1, d2;
-    if constexpr (P == Q::pressure) {
-      d1 = a.p_T();
-      d2 = b.p_T();
-    } else {
-      d1 = a.g_T();
-      d2 = b.g_T();
-    }
-    g.beta = R(0.5) * ((f11 - a.T * d1) + (f22 - b.T * d2));
+    const R t1 = fall(0, 3), t2 = fall(1, 3), rt1 = fall(0, 4), rt2 = fall(1, 4);  // H_T, H_rhoT
+    pb = R(0.5) * ((p11 - a.T * (a.rho * a.rho * rt1)) + (p22 - b.T * (b.rho * b.rho * rt2)));
+    gb = R(0.5) * ((g11 - a.T * (t1 + a.rho * rt1)) + (g22 - b.T * (t2 + b.rho * rt2)));
   }
-  return g;
+  rho_mean = pd / gd;
+  e_mean = gb - pb / rho_mean;
 }
 
-// LTEHelmholtzEOS.hpp:386-397.  In FP64 the two discrete gradients are
-// taken in separate passes of a loop that is not unrolled: written one after
-// the other they share their cell evaluations, which keeps both gradients'
-// table values live at once (about 590 registers, spilled to scratch); apart
-// they fit the register file (256 VGPRs + 238 AGPRs in the 3-D p = 3 RHS
-// kernel, no scratch), and the RHS kernel runs 1.3x faster although the
-// shared evaluations are repeated.  Same arithmetic, same results.
-template <typename R>
-__device__ __forceinline__ void thermodynamic_means(const View &v, const Eval<R> &l, const Eval<R> &r, R &rho_mean,
-                                                    R &e_mean) {
-  Gradient<R> p, g;
-  if constexpr (sizeof(R) == sizeof(double)) {
-#pragma unroll 1
-    for (int k = 0; k < 2; ++k) {
-      if (k == 0) p = discrete_gradient<Q::pressure>(v, l, r);
-      else g = discrete_gradient<Q::gibbs>(v, l, r);
-    }
-  } else {
-    p = discrete_gradient<Q::pressure>(v, l, r);
-    g = discrete_gradient<Q::gibbs>(v, l, r);
-  }
-  rho_mean = p.density / g.density;
-  e_mean = g.beta - p.beta / rho_mean;
-}
-
-// LTEECFlux.hpp:11-85 on evaluated endpoints (p and, for faces, c per
-// endpoint); pd1, pd2: the pressures of the momentum flux's pressure term
-// (p less a constant background in the mixed-precision form, which the
-// divergence does not see; p itself in FP64)
+// LTEECFlux.hpp:11-85 from the entropy-conserving means, the endpoints'
+// states and pressures and, for faces, sound speeds; pd1, pd2: the pressures
+// of the momentum flux's pressure term (p less a constant background in the
+// mixed-precision form, which the divergence does not see; p itself in FP64)
 template <int DIM, bool FACE, typename R>
-__device__ __forceinline__ void lteec_flux(const View &v, const R *q1, const R *q2, const Eval<R> &s1,
-                                           const Eval<R> &s2, R p1, R p2, R c1, R c2, const R *dir, R *F,
-                                           R pd1, R pd2) {
-  R rho_m, e_m;
-  thermodynamic_means(v, s1, s2, rho_m, e_m);
+__device__ __forceinline__ void lteec_flux(R rho_m, R e_m, const R *q1, const R *q2, R p1, R p2, R c1, R c2,
+                                           const R *dir, R *F, R pd1, R pd2) {
   const R pm = R(0.5) * (pd1 + pd2);
   const R ir1 = R(1.0) / q1[0], ir2 = R(1.0) / q2[0];
   R vn = 0, ck = 0, pw = 0, v1n = 0, v2n = 0, n2 = 0;
@@ -431,12 +547,6 @@ __device__ __forceinline__ void lteec_flux(const View &v, const R *q1, const R *
   }
   F[DIM + 1] = mass * (e_m + ck) + pw - diss * (q2[DIM + 1] - q1[DIM + 1]);
 }
-template <int DIM, bool FACE, typename R>
-__device__ __forceinline__ void lteec_flux(const View &v, const R *q1, const R *q2, const Eval<R> &s1,
-                                           const Eval<R> &s2, R p1, R p2, R c1, R c2, const R *dir, R *F) {
-  lteec_flux<DIM, FACE>(v, q1, q2, s1, s2, p1, p2, c1, c2, dir, F, p1, p2);
-}
-
 // Temperature and table cell of every node of a state (one lane per node):
 // the recovery of state_eval, done once per node and stage, for the RHS
 // kernel's staged nodes and its neighbours' face points.
@@ -472,6 +582,28 @@ __global__ void __launch_bounds__(256) k_lte_node_pcg(const double *U, long long
   v.node_p[t] = ev.pressure();
   v.node_c[t] = sqrt(ev.c2());
   if (v.node_g) v.node_g[t] = ev.cp() / ev.cv();
+}
+
+// After k_lte_nodes, for LTEEC: each node's H and its derivatives in the
+// arithmetic type of the pair fluxes, its sound speed and, in the mixed form,
+// its pressure (both FP64), once per node instead of in each of the node's
+// 9 pairs and 1.5 face points per direction and side (3-D p = 3).
+template <typename R>
+__global__ void __launch_bounds__(256) k_lte_node_rec(const double *U, long long Ntot, View v) {
+  const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (t >= Ntot) return;
+  const double rho = U[t], T = v.node_T[t];
+  const int cell = v.node_cell[t];
+  const Eval<double> ev = at_packed<double>(v, rho, T, cell);
+  v.node_c[t] = sqrt(ev.c2());
+  const Eval<R> er = at_packed<R>(v, R(rho), R(T), cell);
+  if constexpr (sizeof(R) != sizeof(double)) v.node_p[t] = ev.pressure();
+  R *o = static_cast<R *>(v.node_rec) + t;
+  o[0] = er.H();
+  o[Ntot] = er.template H<1, 0>();
+  o[2 * Ntot] = er.template H<2, 0>();
+  o[3 * Ntot] = er.template H<0, 1>();
+  o[4 * Ntot] = er.template H<1, 1>();
 }
 
 // ---- the viscous path (LTEGasModel<LTEHelmholtzGasEOS, LTETransport>,

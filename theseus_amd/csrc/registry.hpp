@@ -147,7 +147,10 @@ struct OrdersRegistrar {
 
 template <typename R, int DIM, int P, bool VISC = false, int FX = LTE_FLUX_LTEEC>
 void launch_rhs_lte(const RHSArgs &a, int nb, hipStream_t s) {
-  hipLaunchKernelGGL((k_rhs_lte<R, DIM, P, VISC, FX>), dim3(nb), dim3(Shape<DIM, P>::TPB), 0, s, a);
+  if constexpr (FX == LTE_FLUX_LTEEC)
+    hipLaunchKernelGGL((k_rhs_lteec<R, DIM, P, VISC>), dim3(nb), dim3(Shape<DIM, P>::TPB), 0, s, a);
+  else
+    hipLaunchKernelGGL((k_rhs_lte<R, DIM, P, VISC, FX>), dim3(nb), dim3(Shape<DIM, P>::TPB), 0, s, a);
 }
 template <typename R, int DIM, int P>
 void launch_ns_grad_lte(const RHSArgs &a, int nb, hipStream_t s) {
@@ -162,7 +165,12 @@ template <int DIM>
 void launch_lte_nodes(const RHSArgs &a, int, hipStream_t s) {
   const dim3 grid((unsigned)((a.Ntot + 255) / 256));
   hipLaunchKernelGGL((lte::k_lte_nodes<DIM>), grid, dim3(256), 0, s, a.U, a.Ntot, a.lte);
-  if (a.lte.node_p) hipLaunchKernelGGL((lte::k_lte_node_pcg<DIM>), grid, dim3(256), 0, s, a.U, a.Ntot, a.lte);
+  if (a.lte.node_rec && a.lte.rec32)
+    hipLaunchKernelGGL((lte::k_lte_node_rec<float>), grid, dim3(256), 0, s, a.U, a.Ntot, a.lte);
+  else if (a.lte.node_rec)
+    hipLaunchKernelGGL((lte::k_lte_node_rec<double>), grid, dim3(256), 0, s, a.U, a.Ntot, a.lte);
+  else if (a.lte.node_p)
+    hipLaunchKernelGGL((lte::k_lte_node_pcg<DIM>), grid, dim3(256), 0, s, a.U, a.Ntot, a.lte);
 }
 
 template <int DIM, int P>

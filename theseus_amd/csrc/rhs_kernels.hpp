@@ -276,6 +276,7 @@ template <int Np, int ND>
 struct StagedIndex {
   static constexpr int size = kLdsPad ? ND + ND / Np : ND;
   __host__ __device__ static constexpr int at(int n) { return kLdsPad ? n + n / Np : n; }
+  __host__ __device__ static constexpr int node(int s) { return kLdsPad ? s - s / (Np + 1) : s; }  // inverse of at
 };
 
 // Flux scratch of the volume phase of one workgroup.  The pair list is
