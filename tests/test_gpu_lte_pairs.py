@@ -88,3 +88,33 @@ def test_lteec_outside_the_table_is_nan(oracle):
     touched = {21} | {int(v) for v in mesh.face_neighbor.reshape(64, 6)[21]}
     rest = [e for e in range(64) if e not in touched]
     assert np.array_equal(got[:, rest], ref[:, rest])
+
+
+# The recovery's cell searches on grids of each kind: logarithmic (the
+# workload's), uniform, two cells in a direction, and one whose cells crowd
+# into few buckets (the searches then bisect).
+GRIDS = {
+    "log": dict(nx=40, ny=300),
+    "uniform": dict(nx=50, ny=70, rho=(0.01, 1.0), rho_dist="uniform", T_dist="uniform"),
+    "tiny": dict(nx=3, ny=3, rho=(0.05, 0.3), T=(2000.0, 6000.0)),
+    "crowded": dict(nx=600, ny=64, rho=(1e-30, 1.0), rho_dist="uniform"),
+}
+
+
+@pytest.mark.parametrize("flux", ["lteec", "hll"])
+@pytest.mark.parametrize("grid", list(GRIDS))
+def test_recovery_on_grids(oracle, grid, flux):
+    import dataclasses
+
+    from theseus_amd import _abi as A
+    from theseus_amd.lte import synthetic_table
+
+    rt, mesh, _, rho, T, vel = _setup(3, 3, 3, 0.3, 0.2, 12)
+    if flux == "hll":
+        rt = dataclasses.replace(rt, volume_flux=A.VOLUME_CENTRAL, surface_flux=A.SURFACE_HLL)
+    table = synthetic_table(**GRIDS[grid])
+    ora = _oracle(oracle, rt, mesh, table)
+    U = _state(ora, rho, T, vel)
+    got = _mult(rt, mesh, table, U)
+    assert np.isfinite(got).all()
+    assert rel_l2(got, ora.rhs(U)) <= 1e-12

@@ -473,7 +473,9 @@ struct theseus_rhs {
   int *d_ltecell = nullptr;   // per node: its table cell
   double *d_ltepcg = nullptr; // per node: pressure, sound speed (, gamma); LTEEC: sound speed (, pressure)
   void *d_lterec = nullptr;   // LTEEC, per node: H and its derivatives
-  void *d_ltecells = nullptr; // LTEEC: the table's cell records
+  double *d_ltecells = nullptr;             // the table's cell records
+  float *d_ltecells32 = nullptr;            // mixed LTEEC: in FP32
+  unsigned short *d_ltebuckets = nullptr;   // cell searches' bucket tables
   BasisArgs basis;
   GasC<double> gas;
   GasC<float> gas32;
@@ -745,6 +747,79 @@ static int scratch_for_current_device(double **out) {
   return THESEUS_OK;
 }
 
+// Buckets of one grid (lte::Buckets): kBuckets cells of lower bucket edges
+// appended to `tab`.  A grid whose cells crowd into few buckets (more than 8
+// steps from an edge's cell), or too fine for 16-bit cells, keeps the bisection.
+static constexpr int kBuckets = 4096;
+static bool grid_buckets(const double *g, int n, lte::Buckets &b, std::vector<unsigned short> &tab) {
+  if (n > 65536) return false;
+  auto high = [](double x) {
+    uint64_t u;
+    std::memcpy(&u, &x, sizeof u);
+    return (unsigned)(u >> 32);
+  };
+  b.count = kBuckets;
+  b.positive = g[0] > 0;
+  b.base = b.positive ? high(g[0]) : 0;
+  b.x0 = g[0];
+  b.scale = kBuckets / (g[n - 1] - g[0]);
+  if (b.positive)
+    while (((high(g[n - 1]) - b.base) >> b.shift) >= (unsigned)kBuckets) ++b.shift;
+  auto edge = [&](int k) {
+    if (!b.positive) return b.x0 + k / b.scale;
+    const uint64_t u = (uint64_t)(b.base + ((unsigned)k << b.shift)) << 32;
+    double x;
+    std::memcpy(&x, &u, sizeof x);
+    return x;
+  };
+  auto cell = [&](double x) {
+    return (int)std::min<std::ptrdiff_t>(std::max<std::ptrdiff_t>(std::upper_bound(g, g + n, x) - g - 1, 0), n - 2);
+  };
+  if (!std::isfinite(b.scale)) return false;
+  std::vector<unsigned short> own(kBuckets);
+  int prev = 0;
+  for (int k = 0; k < kBuckets; ++k) {
+    const double x = edge(k);
+    const int c = std::isfinite(x) ? cell(x) : n - 2;
+    if (c - prev > 8) return false;
+    own[k] = (unsigned short)c;
+    prev = c;
+  }
+  if (n - 2 - prev > 8) return false;
+  tab.insert(tab.end(), own.begin(), own.end());
+  return true;
+}
+
+// The cell records and the grids' buckets of a handle's table, from the
+// planes and grids already on the device.
+static int lte_lookups(theseus_rhs *h, const theseus_lte_table *lt) {
+  const size_t ncell = (size_t)lt->nx * lt->ny;
+  const dim3 grid((unsigned)((ncell + 255) / 256));
+  int rc = upload<double>(&h->d_ltecells, nullptr, lte::kCellStride * ncell);
+  if (rc) return rc;
+  hipLaunchKernelGGL(lte::k_lte_cells<double>, grid, dim3(256), 0, nullptr, h->ltev, h->d_ltecells);
+  if (h->pm && h->lfx == LTE_FLUX_LTEEC) {
+    if ((rc = upload<float>(&h->d_ltecells32, nullptr, lte::kCellStride * ncell))) return rc;
+    hipLaunchKernelGGL(lte::k_lte_cells<float>, grid, dim3(256), 0, nullptr, h->ltev, h->d_ltecells32);
+  }
+  HIP_TRY(hipGetLastError());
+  h->ltev.cells64 = h->d_ltecells;
+  h->ltev.cells32 = h->d_ltecells32;
+  std::vector<unsigned short> tab;
+  const double *grids[3] = {lt->rho_grid, lt->T_grid, lt->e_grid};
+  const int counts[3] = {lt->nx, lt->ny, lt->ny};
+  lte::Buckets *b[3] = {&h->ltev.brho, &h->ltev.bT, &h->ltev.be};
+  int at[3];
+  for (int g = 0; g < 3; ++g) {
+    at[g] = (int)tab.size();
+    if (!grid_buckets(grids[g], counts[g], *b[g], tab)) at[g] = -1;
+  }
+  if (!tab.empty() && (rc = upload(&h->d_ltebuckets, tab.data(), tab.size()))) return rc;
+  for (int g = 0; g < 3; ++g) b[g]->cell = at[g] < 0 ? nullptr : h->d_ltebuckets + at[g];
+  HIP_TRY(hipStreamSynchronize(nullptr));
+  return THESEUS_OK;
+}
+
 extern "C" {
 
 const char *theseus_last_error(void) { return g_last_error.c_str(); }
@@ -914,33 +989,22 @@ static int create_impl(const theseus_case_desc *desc, const theseus_lte_table *l
       h->ltev.planes32 = h->d_lte32;
     }
     if (lfx == LTE_FLUX_LTEEC) {
-      // node arrays (sound speed, and in the mixed form pressure, in FP64; H
-      // and its derivatives in the pair fluxes' type) and the cell records
-      const size_t rsz = h->pm ? sizeof(float) : sizeof(double);
-      char *rec = nullptr, *cells = nullptr;
+      // node arrays: sound speed (and in the mixed form pressure) in FP64, H
+      // and its derivatives in the pair fluxes' type
+      char *rec = nullptr;
       if ((rc = upload<double>(&h->d_ltepcg, nullptr, (h->pm ? 2 : 1) * (size_t)h->Ntot)) ||
-          (rc = upload<char>(&rec, nullptr, 5 * rsz * h->Ntot)) ||
-          (rc = upload<char>(&cells, nullptr, lte::kCellStride * rsz * nx * ny))) {
-        hipFree(rec);
+          (rc = upload<char>(&rec, nullptr, 5 * (h->pm ? sizeof(float) : sizeof(double)) * h->Ntot))) {
         theseus_rhs_destroy(h);
         return rc;
       }
       h->d_lterec = rec;
-      h->d_ltecells = cells;
       h->ltev.node_c = h->d_ltepcg;
       h->ltev.node_p = h->pm ? h->d_ltepcg + h->Ntot : nullptr;
       h->ltev.node_rec = rec;
-      h->ltev.rec32 = h->pm;
-      const dim3 grid((unsigned)((nx * ny + 255) / 256));
-      if (h->pm) hipLaunchKernelGGL(lte::k_lte_cells<float>, grid, dim3(256), 0, nullptr, h->ltev, (float *)cells);
-      else hipLaunchKernelGGL(lte::k_lte_cells<double>, grid, dim3(256), 0, nullptr, h->ltev, (double *)cells);
-      hipError_t le = hipGetLastError();
-      if (le == hipSuccess) le = hipStreamSynchronize(nullptr);
-      if (le != hipSuccess) {
-        theseus_rhs_destroy(h);
-        return fail(THESEUS_ERR_DEVICE, std::string("LTE cell records: ") + hipGetErrorString(le));
-      }
-      h->ltev.cells = cells;
+    }
+    if ((rc = lte_lookups(h, lt))) {
+      theseus_rhs_destroy(h);
+      return rc;
     }
   }
   if (d.elem_orient) {
@@ -1038,6 +1102,8 @@ int theseus_rhs_destroy(theseus_rhs *h) {
   hipFree(h->d_ltepcg);
   hipFree(h->d_lterec);
   hipFree(h->d_ltecells);
+  hipFree(h->d_ltecells32);
+  hipFree(h->d_ltebuckets);
   hipFree(h->d_stage[0]);
   hipFree(h->d_stage[1]);
   hipFree(h->d_rates);

@@ -16,6 +16,8 @@
 
 #include <hip/hip_runtime.h>
 
+#include <type_traits>
+
 // No multiply-add contraction in the table arithmetic: the Hermite sums and
 // the thermodynamic combinations built on them (c^2, the divided differences)
 // cancel strongly, and fusing changes their rounding enough to move the
@@ -27,27 +29,40 @@
 namespace thx {
 namespace lte {
 
+// Cell search in an increasing grid: cell[key(x)] is the cell of the lower
+// edge of x's bucket, from which the cell of x is at most a few steps away.
+// The key of a positive grid is linear in the high word of x's
+// bit pattern, piecewise linear in log x; of another grid, linear in x.
+struct Buckets {
+  const unsigned short *cell = nullptr;
+  int count = 0, shift = 0, positive = 0;
+  unsigned base = 0;
+  double x0 = 0, scale = 0;
+};
+
 struct View {
   int nx = 0, ny = 0;
   const double *rho = nullptr, *T = nullptr, *e = nullptr;  // grids
   const double *planes = nullptr;                           // 6 * nx * ny: H, H_rho, H_T, H_rhoT, mu, lambda
   const float *planes32 = nullptr;                          // the planes rounded to FP32 (mixed precision)
   const double *inv = nullptr;                              // nx * ny temperature guesses
+  // bucket tables of the grids (Buckets), for cell searches by a lookup
+  // instead of a bisection; an empty one means bisect
+  Buckets brho, bT, be;
   // per node of the state being evaluated (written by k_lte_nodes): the
   // recovered temperature and the table cell i | j << 16 (-1 outside)
   double *node_T = nullptr;
   int *node_cell = nullptr;
-  // the Pirozzoli, HLL and LLF pairs: each node's pressure and sound speed
-  // (and, for Pirozzoli, gamma = cp/cv), evaluated by k_lte_nodes; null for LTEEC
+  // and what the flux pair takes at it, where set: pressure, sound speed and
+  // (Pirozzoli) gamma = cp/cv in FP64; for LTEEC the sound speed, H, H_rho,
+  // H_rhorho, H_T and H_rhoT ([5][Ntot] of the pair fluxes' type) and, in the
+  // mixed form, the pressure
   double *node_p = nullptr, *node_c = nullptr, *node_g = nullptr;
-  // LTEEC: the scaled Hermite coefficients of every cell (kCellStride values
-  // of the arithmetic type per cell, k_lte_cells) and, per node, H, H_rho,
-  // H_rhorho, H_T and H_rhoT at its recovered temperature ([5][Ntot] of the
-  // arithmetic type, k_lte_node_rec, which writes node_c too and, in the
-  // mixed form, node_p); null for the other pairs
-  const void *cells = nullptr;
   void *node_rec = nullptr;
-  int rec32 = 0;  // the records' arithmetic type: 0 FP64, 1 FP32
+  // the scaled Hermite coefficients of every cell (kCellStride values per
+  // cell, k_lte_cells), in FP64 and, for the mixed form of LTEEC, in FP32
+  const double *cells64 = nullptr;
+  const float *cells32 = nullptr;
   // viscosity of the Navier-Stokes form: the mu plane, or Sutherland's law
   // mu0 (T0 + Ts) (T/T0)^1.5 / (T + Ts) when sutherland is set
   int sutherland = 0;
@@ -70,6 +85,32 @@ __device__ __forceinline__ int find_cell(const double *grid, int count, double v
     else lo = mid;
   }
   return lo;
+}
+
+// find_cell by the grid's buckets (two dependent loads instead of
+// log2(count)), with the cell's ends
+__device__ __forceinline__ int find_cell(const double *grid, int count, const Buckets &b, double value, double &lo,
+                                         double &hi) {
+  if (!(value >= grid[0]) || !(value <= grid[count - 1])) return -1;
+  int i;
+  if (b.cell) {
+    const int k = b.positive ? (int)(((unsigned)(__double_as_longlong(value) >> 32) - b.base) >> b.shift)
+                             : (int)((value - b.x0) * b.scale);
+    i = b.cell[min(max(k, 0), b.count - 1)];
+  } else {
+    i = find_cell(grid, count, value);
+  }
+  lo = grid[i];
+  hi = grid[i + 1];
+  while (i < count - 2 && value >= hi) {
+    lo = hi;
+    hi = grid[++i + 1];
+  }
+  while (i > 0 && value < lo) {  // rounding of the linear key
+    hi = lo;
+    lo = grid[--i];
+  }
+  return i;
 }
 
 template <int D, typename R>
@@ -270,8 +311,8 @@ __device__ __forceinline__ double temperature_from_energy(const View &v, double 
 
 // One cell's record (index j*nx + i): the 16 Hermite coefficients in
 // evaluate()'s order -- per corner (rho side, then T side) H, H_rho wr,
-// H_T wt, (H_rhoT wr) wt -- then wr, wt and the reciprocals of wr, wt, wr wr
-// and wr wt; two values of padding keep records on 64-byte lines.  A pair
+// H_T wt, (H_rhoT wr) wt -- then wr, wt and the reciprocals of wr, wt, wr wr,
+// wr wt and wt wt; one value of padding keeps FP64 records on 64-byte lines.  A pair
 // reads one or two records of consecutive values instead of 32 values strided
 // over four planes and four grid points, with the scalings already applied.
 constexpr int kCellStride = 24;
@@ -300,6 +341,12 @@ __global__ void __launch_bounds__(256) k_lte_cells(View v, R *out) {
   o[19] = R(1) / c.wt;
   o[20] = R(1) / (c.wr * c.wr);
   o[21] = R(1) / (c.wr * c.wt);
+  o[22] = R(1) / (c.wt * c.wt);
+}
+template <typename R>
+__device__ __forceinline__ const R *cells_of(const View &v) {
+  if constexpr (sizeof(R) == sizeof(double)) return v.cells64;
+  else return v.cells32;
 }
 
 // n / d with y the correctly rounded 1 / d: in FP64 the quotient estimate
@@ -419,8 +466,8 @@ __device__ __forceinline__ void thermodynamic_means(const View &v, const PairNod
   if (dd || bd) {
     const int ia = a.cell & 0xFFFF, ja = a.cell >> 16, ib = b.cell & 0xFFFF, jb = b.cell >> 16;
     const bool same = a.cell == b.cell;
-    const R *ca = static_cast<const R *>(v.cells) + (size_t)(jb * v.nx + ia) * kCellStride;
-    const R *cb = static_cast<const R *>(v.cells) + (size_t)(ja * v.nx + ib) * kCellStride;
+    const R *ca = cells_of<R>(v) + (size_t)(jb * v.nx + ia) * kCellStride;
+    const R *cb = cells_of<R>(v) + (size_t)(ja * v.nx + ib) * kCellStride;
     const Basis4<R> dt = dbasis4<0, R>(a.eta, b.eta);
     R c[16], P[16];
     R hx, gx, hdt_a, gdt_a, hy, gy, hdt_b, gdt_b;
@@ -547,10 +594,26 @@ __device__ __forceinline__ void lteec_flux(R rho_m, R e_m, const R *q1, const R 
   }
   F[DIM + 1] = mass * (e_m + ck) + pw - diss * (q2[DIM + 1] - q1[DIM + 1]);
 }
-// Temperature and table cell of every node of a state (one lane per node):
-// the recovery of state_eval, done once per node and stage, for the RHS
-// kernel's staged nodes and its neighbours' face points.
-template <int DIM>
+// What k_lte_nodes leaves per node: the temperature and cell alone (the
+// stability estimate), with what LTEEC takes at a node, or with what the
+// other pairs take (View::node_*).
+enum NodeOut { NODE_T = 0, NODE_LTEEC = 1, NODE_PC = 2 };
+
+// Temperature and table cell of every node of a state and the flux pair's
+// node values there, one lane per node, once per node and stage for the RHS
+// kernel's staged nodes and its neighbours' face points.  The recovery is
+// temperature_from_energy (LTEHelmholtzEOS.hpp:151-223) with its searches and
+// sums arranged for the loop: the density cell is found once, a temperature
+// cell only when the iterate leaves the last one, and the 16 products of the
+// cell's coefficients with the density basis are kept until then, so that an
+// iteration is three sums of 16 products; the operations that round are its
+// own, in its order.  The node values follow in the same kernel, where the
+// cell's record is at hand.  Latency of the dependent lookups (state, bucket,
+// inverse table, bucket, record) at 4 to 5 waves per SIMD bounds it.  At 24^3
+// elements, p = 3 (884,736 nodes): 46 us with LTEEC's values, 44 us with the
+// other pairs', against 72 us for the recovery alone with both cells bisected
+// in every iteration and 39 (22) us for the values in a pass of their own.
+template <int DIM, int OUT, typename R = double>
 __global__ void __launch_bounds__(256) k_lte_nodes(const double *U, long long Ntot, View v) {
   const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
   if (t >= Ntot) return;
@@ -562,48 +625,115 @@ __global__ void __launch_bounds__(256) k_lte_nodes(const double *U, long long Nt
   for (int d = 0; d < DIM; ++d) m2 += q[1 + d] * q[1 + d];
   const double rho = q[0];
   const double e = (q[DIM + 1] - 0.5 * m2 / rho) / rho;
-  const double T = temperature_from_energy(v, rho, e);
-  const int i = find_cell(v.rho, v.nx, rho);
-  const int j = find_cell(v.T, v.ny, T);
+  double rlo = 0, rhi = 1, elo = 0, ehi = 1;
+  const int i = find_cell(v.rho, v.nx, v.brho, rho, rlo, rhi);
+  const int ie = find_cell(v.e, v.ny, v.be, e, elo, ehi);
+  double T = __builtin_nan(""), xi = T;
+  int j = -1;         // cell of the last evaluated temperature, [Tlo, Thi) (closed at the grid's end)
+  double Tlo = 0, Thi = 0, wt = 1, iwt = 1, iwtt = 1;
+  const double *rec = v.cells64;
+  double P[16];       // its coefficients times the density basis
+  const double Tmin = v.T[0], Tmax = v.T[v.ny - 1];
+  // makes j, Tlo, Thi and rec those of the temperature x; false outside the grid
+  auto locate = [&](double x) {
+    if (j >= 0 && x >= Tlo && x < Thi) return true;
+    const int n = find_cell(v.T, v.ny, v.bT, x, Tlo, Thi);
+    if (n < 0) return false;
+    j = n;
+    rec = v.cells64 + (size_t)(j * v.nx + i) * kCellStride;
+    wt = rec[17];
+    iwt = rec[19];
+    iwtt = rec[22];
+    return true;
+  };
+  auto rho_rows = [&](auto D) {
+    constexpr int K = decltype(D)::value;
+    cell_row(rec, basis4<K, double>(xi), P);
+  };
+  if (i >= 0 && ie >= 0) {
+    xi = (rho - rlo) / (rhi - rlo);
+    const double y = (e - elo) / (ehi - elo);
+    const double *p = v.inv + ie * v.nx + i;
+    const double lower = p[0] + xi * (p[1] - p[0]);
+    const double upper = p[v.nx] + xi * (p[v.nx + 1] - p[v.nx]);
+    double x = lower + y * (upper - lower);
+    int last = -1;
+    for (int it = 0; it < 100; ++it) {
+      if (!locate(x)) break;
+      if (j != last) {
+        rho_rows(std::integral_constant<int, 0>{});
+        last = j;
+      }
+      const double eta = div_by(x - Tlo, wt, iwt);
+      const double h = cell_dot(P, basis4<0, double>(eta));
+      const double hT = div_by(cell_dot(P, basis4<1, double>(eta)), wt, iwt);
+      const double hTT = div_by(cell_dot(P, basis4<2, double>(eta)), wt * wt, iwtt);
+      const double cv = -x * hTT, guess = h - x * hT;
+      if (!(cv > 0) || !isfinite(guess)) break;
+      const double step = (e - guess) / cv;
+      const double next = x + step;
+      const bool inside = isfinite(next) && next >= Tmin && next <= Tmax;
+      if (fabs(step) <= 1e-9 + 1e-12 * x) {
+        T = next < Tmin ? Tmin : (next > Tmax ? Tmax : next);
+        break;
+      }
+      x = next;
+      if (!inside) break;
+    }
+  }
+  const bool ok = i >= 0 && locate(T);
   v.node_T[t] = T;
-  v.node_cell[t] = (i < 0 || j < 0) ? -1 : (i | (j << 16));
-}
-
-// After k_lte_nodes, for the pairs other than LTEEC: each node's pressure,
-// sound speed and (when node_g is set) gamma = cp/cv at its recovered
-// temperature.  A pass of its own: the evaluation needs about 160 registers,
-// which inside the recovery would hold the Newton iterations to 3 waves per
-// SIMD instead of 7.
-template <int DIM>
-__global__ void __launch_bounds__(256) k_lte_node_pcg(const double *U, long long Ntot, View v) {
-  const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= Ntot) return;
-  const Eval<double> ev = at_packed<double>(v, U[t], v.node_T[t], v.node_cell[t]);
-  v.node_p[t] = ev.pressure();
-  v.node_c[t] = sqrt(ev.c2());
-  if (v.node_g) v.node_g[t] = ev.cp() / ev.cv();
-}
-
-// After k_lte_nodes, for LTEEC: each node's H and its derivatives in the
-// arithmetic type of the pair fluxes, its sound speed and, in the mixed form,
-// its pressure (both FP64), once per node instead of in each of the node's
-// 9 pairs and 1.5 face points per direction and side (3-D p = 3).
-template <typename R>
-__global__ void __launch_bounds__(256) k_lte_node_rec(const double *U, long long Ntot, View v) {
-  const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= Ntot) return;
-  const double rho = U[t], T = v.node_T[t];
-  const int cell = v.node_cell[t];
-  const Eval<double> ev = at_packed<double>(v, rho, T, cell);
-  v.node_c[t] = sqrt(ev.c2());
-  const Eval<R> er = at_packed<R>(v, R(rho), R(T), cell);
-  if constexpr (sizeof(R) != sizeof(double)) v.node_p[t] = ev.pressure();
-  R *o = static_cast<R *>(v.node_rec) + t;
-  o[0] = er.H();
-  o[Ntot] = er.template H<1, 0>();
-  o[2 * Ntot] = er.template H<2, 0>();
-  o[3 * Ntot] = er.template H<0, 1>();
-  o[4 * Ntot] = er.template H<1, 1>();
+  v.node_cell[t] = ok ? (i | (j << 16)) : -1;
+  if constexpr (OUT != NODE_T) {
+    // a node outside the table reads cell (0, 0) at NaN coordinates
+    double eta = __builtin_nan("");
+    if (ok) {
+      eta = div_by(T - Tlo, wt, iwt);
+    } else {
+      xi = eta;
+      rec = v.cells64;
+    }
+    const double wr = rec[16];
+    const Basis4<double> t0 = basis4<0, double>(eta), t1 = basis4<1, double>(eta);
+    rho_rows(std::integral_constant<int, 0>{});
+    const double hTT = div_by(cell_dot(P, basis4<2, double>(eta)), wt * wt, iwtt);
+    double h = 0, hT = 0;
+    if constexpr (OUT == NODE_LTEEC && sizeof(R) == sizeof(double)) {
+      h = cell_dot(P, t0);
+      hT = div_by(cell_dot(P, t1), wt, iwt);
+    }
+    rho_rows(std::integral_constant<int, 1>{});
+    const double hr = div_by(cell_dot(P, t0), wr, rec[18]);
+    const double m = div_by(cell_dot(P, t1), wr * wt, rec[21]);
+    rho_rows(std::integral_constant<int, 2>{});
+    const double hrr = div_by(cell_dot(P, t0), wr * wr, rec[20]);
+    const double p_rho = 2 * rho * hr + rho * rho * hrr;
+    v.node_c[t] = sqrt(p_rho - rho * rho * m * m / hTT);
+    if constexpr (OUT == NODE_PC) {
+      v.node_p[t] = rho * rho * hr;
+      if (v.node_g) {
+        const double cv = -T * hTT;
+        v.node_g[t] = (cv + T * rho * rho * m * m / p_rho) / cv;
+      }
+    } else {
+      R *o = static_cast<R *>(v.node_rec) + t;
+      if constexpr (sizeof(R) == sizeof(double)) {
+        o[0] = h;
+        o[Ntot] = hr;
+        o[2 * Ntot] = hrr;
+        o[3 * Ntot] = hT;
+        o[4 * Ntot] = m;
+      } else {
+        v.node_p[t] = rho * rho * hr;
+        const Eval<R> er = at_packed<R>(v, R(rho), R(T), ok ? (i | (j << 16)) : -1);
+        o[0] = er.H();
+        o[Ntot] = er.template H<1, 0>();
+        o[2 * Ntot] = er.template H<2, 0>();
+        o[3 * Ntot] = er.template H<0, 1>();
+        o[4 * Ntot] = er.template H<1, 1>();
+      }
+    }
+  }
 }
 
 // ---- the viscous path (LTEGasModel<LTEHelmholtzGasEOS, LTETransport>,

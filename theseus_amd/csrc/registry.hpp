@@ -52,7 +52,7 @@ struct OrdersKernels {
 // Each instantiation file registers the fields it sets (the rest null).
 struct LteKernels {
   RHSLaunch rhs[4][2] = {};        // Euler
-  RHSLaunch nodes = nullptr;       // temperature recovery per node (k_lte_nodes, FP64), before rhs
+  RHSLaunch nodes = nullptr;       // temperature recovery and node values (k_lte_nodes, FP64), before rhs
   RHSLaunch ns_grad[2] = {};       // Navier-Stokes pass 1 of the tabulated gas (after nodes)
   RHSLaunch ns[4][2] = {};         // Navier-Stokes pass 2 (after ns_grad)
   RHSLaunch pref = nullptr;        // mixed precision: the background pressure of a state
@@ -164,13 +164,14 @@ void launch_pref_lte(const RHSArgs &a, int, hipStream_t s) {
 template <int DIM>
 void launch_lte_nodes(const RHSArgs &a, int, hipStream_t s) {
   const dim3 grid((unsigned)((a.Ntot + 255) / 256));
-  hipLaunchKernelGGL((lte::k_lte_nodes<DIM>), grid, dim3(256), 0, s, a.U, a.Ntot, a.lte);
-  if (a.lte.node_rec && a.lte.rec32)
-    hipLaunchKernelGGL((lte::k_lte_node_rec<float>), grid, dim3(256), 0, s, a.U, a.Ntot, a.lte);
+  if (a.lte.node_rec && a.lte.cells32)
+    hipLaunchKernelGGL((lte::k_lte_nodes<DIM, lte::NODE_LTEEC, float>), grid, dim3(256), 0, s, a.U, a.Ntot, a.lte);
   else if (a.lte.node_rec)
-    hipLaunchKernelGGL((lte::k_lte_node_rec<double>), grid, dim3(256), 0, s, a.U, a.Ntot, a.lte);
+    hipLaunchKernelGGL((lte::k_lte_nodes<DIM, lte::NODE_LTEEC>), grid, dim3(256), 0, s, a.U, a.Ntot, a.lte);
   else if (a.lte.node_p)
-    hipLaunchKernelGGL((lte::k_lte_node_pcg<DIM>), grid, dim3(256), 0, s, a.U, a.Ntot, a.lte);
+    hipLaunchKernelGGL((lte::k_lte_nodes<DIM, lte::NODE_PC>), grid, dim3(256), 0, s, a.U, a.Ntot, a.lte);
+  else
+    hipLaunchKernelGGL((lte::k_lte_nodes<DIM, lte::NODE_T>), grid, dim3(256), 0, s, a.U, a.Ntot, a.lte);
 }
 
 template <int DIM, int P>

@@ -7,14 +7,14 @@
 // last three take the gas's pressure, sound speed and cp/cv at each node
 // from the table at its recovered temperature.  Same element-per-
 // workgroup structure as k_rhs: the element's temperatures are recovered
-// once per node per stage by k_lte_nodes (inverse-table guess + Newton)
-// and staged in LDS with the table cell, so the pair fluxes only evaluate
-// the interpolant; each GLL-line pair is evaluated once; the neighbours' face
-// traces come with their recovered temperatures and cells.  With VISC it is
-// the Navier-Stokes pass 2 of the tabulated gas (periodic meshes): the
-// viscous volume divergence with the own half of the central viscous face
-// flux, and the neighbours' n.Fv, come from k_ns_grad<..., LTE> as for the
-// ideal gas (DGSEMIntegrator.hpp:261-316, 486-622).
+// once per node per stage by k_lte_nodes (inverse-table guess + Newton),
+// with the values of the interpolant there that the flux pair takes; each
+// GLL-line pair is evaluated once; the neighbours' face traces come with
+// their node values.  With VISC it is the Navier-Stokes pass 2 of the
+// tabulated gas (periodic meshes): the viscous volume divergence with the own
+// half of the central viscous face flux, and the neighbours' n.Fv, come from
+// k_ns_grad<..., LTE> as for the ideal gas (DGSEMIntegrator.hpp:261-316,
+// 486-622).
 //
 // R = float is the mixed-precision form: the staged states and the pair and
 // face fluxes (the Itoh-Abe means of the interpolant) in FP32; each node's
@@ -99,7 +99,7 @@ __global__ void __launch_bounds__((Shape<DIM, P>::TPB)) k_rhs_lte(RHSArgs a) {
   meta_load_normals<DIM, EPB, TPB>(a, ebase_blk, mr);
   if (tid < Np * Np) sD2[tid] = R(bD2);
 
-  // ---- stage; pressure and sound speed from k_lte_node_pcg
+  // ---- stage; pressure and sound speed from k_lte_nodes
   meta_store<DIM, EPB, TPB>(mr, sm);
   if (valid) {
 #pragma unroll
@@ -325,12 +325,12 @@ __global__ void __launch_bounds__((Shape<DIM, P>::TPB)) k_rhs_lte(RHSArgs a) {
 }
 
 // The tabulated gas's Euler right-hand side (or Navier-Stokes pass 2) with the
-// LTEEC flux.  Per-node quantities come from k_lte_nodes and k_lte_node_rec; a
+// LTEEC flux.  Per-node quantities come from k_lte_nodes; a
 // pair evaluates only what depends on both endpoints (thermodynamic_means).
 // Bound by FP64 issue: 861 vector instructions a pair, none of which may be
 // contracted (device_lte.hpp), 72.7 M per launch at 24^3 elements, p = 3,
 // which issue in 145 us at the 2.0 GHz the card holds there.  Measured at that size: 218 us
-// (RHS 291 us with the node passes) against 926 us (964 us) when each pair
+// (RHS 234 us with the node pass) against 926 us (964 us) when each pair
 // evaluated both endpoints and the two gradients separately, at one wave per
 // SIMD with 494 registers.
 //
@@ -411,7 +411,7 @@ __attribute__((amdgpu_waves_per_eu(LteecWaves<R, DIM, P, VISC>::value))) k_rhs_l
   if (tid < Np * Np) sD2[tid] = R(bD2);
   meta_store<DIM, EPB, TPB>(mr, sm);
 
-  // a node's or face trace's endpoint from the arrays of k_lte_nodes and k_lte_node_rec
+  // a node's or face trace's endpoint from the arrays of k_lte_nodes
   auto global_node = [&](size_t n, R rho) {
     return lte::pair_node<R>(tv, rho, R(tv.node_T[n]), tv.node_cell[n], rec[n], rec[Ntot + n]);
   };
