@@ -111,25 +111,25 @@ __device__ __forceinline__ bool bc_zero_flux(int type, bool visc) {
   return !visc && (type == BC_NO_SLIP_ADIABATIC || type == BC_NO_SLIP_ISOTHERMAL);
 }
 
-// BR1 boundary jump S_bc - S in entropy variables (ComputeBdrFaceGradFlux,
-// bc_kernels.hpp:32-135); zero for the types without one.
+// BR1 boundary jump S_bc - S of the viscous variables (beta u, -beta)
+// (ComputeBdrFaceGradFlux, bc_kernels.hpp:32-135); zero for the types without one.
 template <typename R, int DIM>
 __device__ __forceinline__ void bc_grad_jump(const GasC<R> &g, int type, const double *data, const R *S, R *jump) {
 #pragma unroll
-  for (int k = 0; k < DIM + 2; ++k) jump[k] = R(0);
+  for (int k = 0; k <= DIM; ++k) jump[k] = R(0);
   if (type == BC_PRESCRIBED_STATE) {
-    R qb[DIM + 2], E[DIM + 2];
+    R qb[DIM + 2], E[DIM + 1];
 #pragma unroll
     for (int k = 0; k < DIM + 2; ++k) qb[k] = R(data[k]);
-    entropy_state<R, DIM>(g, qb, E);
+    viscous_variables<R, DIM>(g, qb, E);
 #pragma unroll
-    for (int k = 0; k < DIM + 2; ++k) jump[k] = E[k] - S[k];
+    for (int k = 0; k <= DIM; ++k) jump[k] = E[k] - S[k];
   } else if (type == BC_NO_SLIP_ADIABATIC || type == BC_NO_SLIP_ISOTHERMAL) {
     // wall velocity at the node's own beta (adiabatic) or at 1/(R T_wall) (isothermal)
-    const R beta = type == BC_NO_SLIP_ADIABATIC ? -S[DIM + 1] : R(1.0 / (double(g.R_gas) * data[DIM]));
+    const R beta = type == BC_NO_SLIP_ADIABATIC ? -S[DIM] : R(1.0 / (double(g.R_gas) * data[DIM]));
 #pragma unroll
-    for (int d = 0; d < DIM; ++d) jump[1 + d] = R(data[d]) * beta - S[1 + d];
-    jump[DIM + 1] = -beta - S[DIM + 1];
+    for (int d = 0; d < DIM; ++d) jump[d] = R(data[d]) * beta - S[d];
+    jump[DIM] = -beta - S[DIM];
   }
 }
 

@@ -706,6 +706,8 @@ static void init_gas(const theseus_case_desc &d, GasC<double> &g, GasC<float> &g
   g.mu = d.mu;
   g.mu_bulk = d.mu_bulk;
   g.R_gas = d.R_gas;
+  g.kappa = g.mu * g.cp * g.PrInverse;
+  g.dTdB = g.gammaM1Inverse * g.gamma / g.cp;
   g32.gamma = (float)g.gamma;
   g32.gammaM1 = (float)g.gammaM1;
   g32.gammaM1Inverse = (float)g.gammaM1Inverse;
@@ -714,6 +716,8 @@ static void init_gas(const theseus_case_desc &d, GasC<double> &g, GasC<float> &g
   g32.mu = (float)g.mu;
   g32.mu_bulk = (float)g.mu_bulk;
   g32.R_gas = (float)g.R_gas;
+  g32.kappa = (float)g.kappa;
+  g32.dTdB = (float)g.dTdB;
 }
 
 // Workgroup partials of the integral measures for callers that cannot

@@ -747,21 +747,16 @@ struct ViscNode {
   R T, mu, kappa;
 };
 
-// Entropy variables ((g - |u|^2/2)/T, u/T, -1/T) of a node whose temperature
-// and cell were recovered (LTEHelmholtzGasEOS.hpp:144-157; the kinetic term
-// is the kinetic energy density over rho, :40-50)
+// The entropy variables the viscous flux depends on, (u/T, -1/T), of a node
+// whose temperature was recovered (LTEHelmholtzGasEOS.hpp:144-157; the first,
+// (g - |u|^2/2)/T, does not enter the conversion to grad u and grad T,
+// :159-171, so g is not evaluated)
 template <int DIM, typename R>
-__device__ __forceinline__ void entropy_state(const View &v, const R *q, R T, int cell, R *E) {
-  const Eval<R> s = at_packed<R>(v, q[0], T, cell);
-  const R beta = 1 / s.T;
-  R m2 = 0;
+__device__ __forceinline__ void viscous_variables(const R *q, R T, R *S) {
+  const R beta = 1 / T;
 #pragma unroll
-  for (int d = 0; d < DIM; ++d) m2 += q[1 + d] * q[1 + d];
-  const R kinetic = R(0.5) * m2 / q[0] / q[0];
-  E[0] = beta * (s.gibbs() - kinetic);
-#pragma unroll
-  for (int d = 0; d < DIM; ++d) E[1 + d] = beta * (q[1 + d] / q[0]);
-  E[DIM + 1] = -beta;
+  for (int d = 0; d < DIM; ++d) S[d] = beta * (q[1 + d] / q[0]);
+  S[DIM] = -beta;
 }
 
 template <int DIM, typename R>

@@ -20,6 +20,8 @@ namespace thx {
 template <typename R>
 struct GasC {
   R gamma, gammaM1, gammaM1Inverse, cp, PrInverse, mu, mu_bulk, R_gas;
+  R kappa;  // conductivity mu cp / Pr (Transport.hpp:19-54)
+  R dTdB;   // gamma / ((gamma - 1) cp) = 1/R: grad T = dTdB (p/rho)^2 grad(-rho/p)
 };
 
 template <typename R, int DIM>
@@ -706,20 +708,29 @@ __device__ __forceinline__ void entropy_state(const GasC<R> &g, const R *q, R *E
   E[DIM + 1] = -beta;
 }
 
-// EOS.hpp:236-263 : gradient of entropy variables -> gradient of (rho, u, p)
+// The entropy variables the viscous flux depends on, (beta u, -beta): EOS.hpp:
+// 236-263 converts the gradient of all of them to that of (rho, u, p) and
+// :159-173 those to grad T, in which the first variable's gradient cancels
+// (grad p = (p/rho) (grad rho + p grad(-beta)), so grad p - (p/rho) grad rho
+// holds grad(-beta) alone).  Leaving it out drops two logarithms a state, a
+// fifth of the contractions, and the rounding of that cancellation.
 template <typename R, int DIM>
-__device__ __forceinline__ void grad_entropy_to_grad_prim(const NodeThermo<R, DIM> &t, const R *q, const R *dE,
-                                                          R *dP) {
-  const R p_over_rho = t.p * t.ir;
-  R drho = R(0);
+__device__ __forceinline__ void viscous_variables(const GasC<R> &g, const R *q, R *S) {
+  const NodeThermo<R, DIM> t = node_thermo<R, DIM>(g, q);
 #pragma unroll
-  for (int d = 0; d < DIM; d++) {
-    dP[1 + d] = p_over_rho * (dE[1 + d] + t.u[d] * dE[DIM + 1]);
-    drho += q[1 + d] * dP[1 + d];
-  }
-  drho = t.rho * dE[0] - dE[DIM + 1] * (t.ke - t.ie) + t.beta * drho;
-  dP[0] = drho;
-  dP[DIM + 1] = p_over_rho * (dP[0] + t.p * dE[DIM + 1]);
+  for (int d = 0; d < DIM; ++d) S[d] = t.beta * t.u[d];
+  S[DIM] = -t.beta;
+}
+
+// One direction's velocity and temperature gradients from those variables'
+// gradient dS
+template <typename R, int DIM>
+__device__ __forceinline__ void viscous_gradients(const GasC<R> &g, const NodeThermo<R, DIM> &t, const R *dS, R *dV,
+                                                  R &dT) {
+  const R p_over_rho = t.p * t.ir;
+#pragma unroll
+  for (int d = 0; d < DIM; d++) dV[d] = p_over_rho * (dS[d] + t.u[d] * dS[DIM]);
+  dT = g.dTdB * (p_over_rho * p_over_rho) * dS[DIM];
 }
 
 // Number of stored viscous-flux components per node: the symmetric stress
@@ -738,21 +749,22 @@ struct VisComp {
 };
 
 // Physical viscous flux, NavierStokesFlux.hpp:160-290 (Cartesian), from the
-// transport coefficients, the velocity u, the temperature gradient gt and the
-// primitive gradients dP[dir][]; writes the unique components in VisComp order.
+// transport coefficients, the velocity u and the gradients of velocity
+// dV[dir][] and temperature dT[dir]; writes the unique components in VisComp
+// order.
 template <typename R, int DIM>
-__device__ __forceinline__ void viscous_flux_core(R mu, R kappa, R mu_bulk, const R *u, const R *gt,
-                                                  const R (*dP)[DIM + 2], R *out) {
+__device__ __forceinline__ void viscous_flux(R mu, R kappa, R mu_bulk, const R *u, const R (*dV)[DIM], const R *dT,
+                                             R *out) {
   R div_vel = R(0);
 #pragma unroll
-  for (int d = 0; d < DIM; ++d) div_vel += dP[d][1 + d];
+  for (int d = 0; d < DIM; ++d) div_vel += dV[d][d];
   R tau[DIM][DIM];
 #pragma unroll
   for (int dir = 0; dir < DIM; ++dir)
 #pragma unroll
     for (int mom = 0; mom < DIM; ++mom) {
-      if (mom == dir) tau[mom][dir] = mu * (R(2) * dP[dir][1 + mom] - mu_bulk * div_vel);
-      else tau[mom][dir] = mu * (dP[dir][1 + mom] + dP[mom][1 + dir]);
+      if (mom == dir) tau[mom][dir] = mu * (R(2) * dV[dir][mom] - mu_bulk * div_vel);
+      else tau[mom][dir] = mu * (dV[dir][mom] + dV[mom][dir]);
     }
 #pragma unroll
   for (int a = 0; a < DIM; ++a)
@@ -760,50 +772,9 @@ __device__ __forceinline__ void viscous_flux_core(R mu, R kappa, R mu_bulk, cons
     for (int b = a; b < DIM; ++b) out[VisComp<DIM>::tau(a, b)] = tau[a][b];
 #pragma unroll
   for (int dir = 0; dir < DIM; ++dir) {
-    R ef = kappa * gt[dir];
+    R ef = kappa * dT[dir];
 #pragma unroll
     for (int mom = 0; mom < DIM; ++mom) ef += u[mom] * tau[mom][dir];
-    out[VisComp<DIM>::en(dir)] = ef;
-  }
-}
-
-// The ideal gas: constant viscosity, kappa = mu cp / Pr (Transport.hpp:19-54)
-// and grad T from the pressure and density gradients (EOS.hpp:159-173,
-// fac = (1/(gamma-1)) / (cv rho), cv = cp/gamma).  The same arithmetic as
-// viscous_flux_core, written out: computing grad T and div u in one loop
-// keeps the FP64 gradient kernel of the 3-D p = 3 case within its registers.
-template <typename R, int DIM>
-__device__ __forceinline__ void viscous_flux(const GasC<R> &g, const NodeThermo<R, DIM> &t, const R (*dP)[DIM + 2],
-                                             R *out) {
-  const R mu = g.mu;
-  const R kappa = g.mu * g.cp * g.PrInverse;
-  const R mu_bulk = g.mu_bulk;
-  const R pressor = t.p * t.ir;
-  const R fac = g.gammaM1Inverse * g.gamma / g.cp * t.ir;
-  R gt[DIM];
-  R div_vel = R(0);
-#pragma unroll
-  for (int d = 0; d < DIM; ++d) {
-    gt[d] = fac * (dP[d][DIM + 1] - pressor * dP[d][0]);
-    div_vel += dP[d][1 + d];
-  }
-  R tau[DIM][DIM];
-#pragma unroll
-  for (int dir = 0; dir < DIM; ++dir)
-#pragma unroll
-    for (int mom = 0; mom < DIM; ++mom) {
-      if (mom == dir) tau[mom][dir] = mu * (R(2) * dP[dir][1 + mom] - mu_bulk * div_vel);
-      else tau[mom][dir] = mu * (dP[dir][1 + mom] + dP[mom][1 + dir]);
-    }
-#pragma unroll
-  for (int a = 0; a < DIM; ++a)
-#pragma unroll
-    for (int b = a; b < DIM; ++b) out[VisComp<DIM>::tau(a, b)] = tau[a][b];
-#pragma unroll
-  for (int dir = 0; dir < DIM; ++dir) {
-    R ef = kappa * gt[dir];
-#pragma unroll
-    for (int mom = 0; mom < DIM; ++mom) ef += t.u[mom] * tau[mom][dir];
     out[VisComp<DIM>::en(dir)] = ef;
   }
 }

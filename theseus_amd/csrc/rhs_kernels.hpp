@@ -13,11 +13,10 @@
 //   4. optionally evaluates the Persson-Peraire indicator and the subcell
 //      FV residual and blends;
 //   5. writes dU (or the fused SSP-RK3 stage combination) once per node.
-// For Navier-Stokes (BR1) a first kernel computes the entropy-variable
-// gradient with its face lift, converts it to primitive gradients and
-// stores only the physical viscous flux (symmetric stress + energy flux,
-// 9 values/node in 3-D); the second kernel is the kernel above plus the
-// viscous volume divergence and the central viscous face term.
+// For Navier-Stokes (BR1) a first kernel computes the gradient of the entropy
+// variables with its face lift, converts it to velocity and temperature
+// gradients and stores the viscous volume divergence and n.Fv at the face
+// points; the second kernel is the kernel above plus those.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -1109,6 +1108,10 @@ __attribute__((amdgpu_waves_per_eu(sizeof(R) == sizeof(double) || BND ? 4 : 5)))
 // plus the element's own half of the central viscous face flux,
 // -0.5 n.Fv lifted with the face weight, and n.Fv at every point of the
 // element's faces for the neighbours' halves (n the canonical area vector).
+// Only the entropy variables the viscous flux depends on are differentiated
+// (viscous_variables): with all of them and their two logarithms per node and
+// face point the FP64 pass took 118 us and 95 VGPRs at 32^3 elements, p = 3,
+// now 92 us and 77; the FP32 pass 67 us, now 60.
 // ---------------------------------------------------------------------------
 // ---------------------------------------------------------------------------
 // Matrix-core line contractions of the gradient pass (FP32, 3-D, p = 3, one
@@ -1159,62 +1162,24 @@ __device__ __forceinline__ void line_contract_dir(const float (*F)[64], const fl
   for (int q = 0; q < 4; ++q) out[q] = DIR == 0 ? c[q] : lane_fetch(src, c[q]);
 }
 
-// All three directions of five fields: out[d][r]; the fifth field's three
-// directions share one product set (rows 0, 1, 2 of its blocks).  Every
-// lane of the wave must call it.
-__device__ __forceinline__ void line_contract_mfma5(const float (*F)[64], const float op[4], int t, float (*out)[5]) {
-  float o[4];
-  line_contract_dir<0>(F, op, t, o);
-#pragma unroll
-  for (int q = 0; q < 4; ++q) out[0][q] = o[q];
-  line_contract_dir<1>(F, op, t, o);
-#pragma unroll
-  for (int q = 0; q < 4; ++q) out[1][q] = o[q];
-  line_contract_dir<2>(F, op, t, o);
-#pragma unroll
-  for (int q = 0; q < 4; ++q) out[2][q] = o[q];
-  const int b = t >> 2, r = t & 3;
-  const int b4 = r == 0 ? mfma_line_base<0>(b) : (r == 1 ? mfma_line_base<1>(b) : mfma_line_base<2>(b));
-  const int s4 = r == 0 ? 1 : (r == 1 ? 4 : 16);
-  mfma_f4 c = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-  for (int l = 0; l < 4; ++l) c = __builtin_amdgcn_mfma_f32_4x4x1f32(r < 3 ? F[4][b4 + s4 * l] : 0.f, op[l], c, 0, 0, 0);
-  out[0][4] = c[0];
-  out[1][4] = lane_fetch(mfma_src_y(t), c[1]);
-  out[2][4] = lane_fetch(mfma_src_z(t), c[2]);
-}
-
-// Occupancy requested for the gradient pass: 5 waves per SIMD for FP64 3-D
-// p = 3 on periodic meshes (at most 96 VGPRs; the LDS allows 5.5), where
-// the allocator would otherwise take 116 and run 4; 8 for its FP32 form
-// with the matrix-core contractions (64 VGPRs, as without them); elsewhere
-// the default.  With the boundary code either would spill.
+// Occupancy requested for the gradient pass: 6 waves per SIMD for FP64 3-D
+// p = 3 on periodic meshes (77 VGPRs; the LDS allows 6); 8 for its FP32 form
+// with the matrix-core contractions (58 VGPRs); elsewhere the default.
 template <typename R, int DIM, int P, int EPBX, bool BND, bool LTE = false>
 struct GradWaves {
   static constexpr bool fits = sizeof(R) == sizeof(double) && DIM == 3 && P == 3 && EPBX == 0 && !BND && !LTE;
-  static constexpr int value = fits ? 5 : (GradMfma<R, DIM, P, EPBX>::on && !BND && !LTE ? 8 : 1);  // 64 VGPRs
+  static constexpr int value = fits ? 6 : (GradMfma<R, DIM, P, EPBX>::on && !BND && !LTE ? 8 : 1);
 };
 
-// The tabulated gas on the BR1 path: the primitive gradient (0, grad u, grad T)
-// from the entropy-variable gradient (LTEHelmholtzGasEOS.hpp:159-171) and the
-// viscous flux with the node's tabulated viscosity and conductivity, grad T
-// taken from the energy slot (grad_temperature, :133-142)
+// The tabulated gas on the BR1 path: grad u and grad T from the gradient of
+// (u/T, -1/T) (LTEHelmholtzGasEOS.hpp:159-171)
 template <typename R, int DIM>
-__device__ __forceinline__ void grad_entropy_to_grad_prim(const lte::ViscNode<DIM, R> &t, const R *, const R *dE,
-                                                          R *dP) {
+__device__ __forceinline__ void viscous_gradients(const GasC<R> &, const lte::ViscNode<DIM, R> &t, const R *dS, R *dV,
+                                                  R &dT) {
   const R T = t.T;
-  dP[0] = R(0);
 #pragma unroll
-  for (int d = 0; d < DIM; ++d) dP[1 + d] = T * dE[1 + d] + T * t.u[d] * dE[DIM + 1];
-  dP[DIM + 1] = T * T * dE[DIM + 1];
-}
-template <typename R, int DIM>
-__device__ __forceinline__ void viscous_flux(const GasC<R> &g, const lte::ViscNode<DIM, R> &t, const R (*dP)[DIM + 2],
-                                             R *out) {
-  R gt[DIM];
-#pragma unroll
-  for (int d = 0; d < DIM; ++d) gt[d] = dP[d][DIM + 1];
-  viscous_flux_core<R, DIM>(t.mu, t.kappa, g.mu_bulk, t.u, gt, dP, out);
+  for (int d = 0; d < DIM; ++d) dV[d] = T * dS[d] + T * t.u[d] * dS[DIM];
+  dT = T * T * dS[DIM];
 }
 
 // LTE: the tabulated gas (periodic meshes); its nodes' temperatures and
@@ -1227,9 +1192,10 @@ __attribute__((amdgpu_waves_per_eu(GradWaves<R, DIM, P, EPBX, BND, LTE>::value))
   constexpr int Np = S::Np, ND = S::NDOF, NF = S::NFP, NQ = S::NEQ, EPB = S::EPB, TPB = S::TPB;
   constexpr int NV = VisComp<DIM>::N;
   constexpr int NVD = DIM + 1;
+  constexpr int NG = DIM + 1;  // variables whose gradient the viscous flux takes (viscous_variables)
   constexpr int NFACE = 2 * DIM * NF;
   constexpr int NFR = (EPB * NFACE + TPB - 1) / TPB;
-  constexpr int NA = EPB * NQ * ND + EPB * NFACE * NQ;  // entropy variables + face jumps
+  constexpr int NA = EPB * NG * ND + EPB * NFACE * NG;  // variables + face jumps
   constexpr int NB = EPB * DIM * NVD * ND;              // contravariant viscous fluxes
   constexpr int NBUF = NA > NB ? NA : NB;
 
@@ -1238,8 +1204,8 @@ __attribute__((amdgpu_waves_per_eu(GradWaves<R, DIM, P, EPBX, BND, LTE>::value))
   __shared__ R sDh[Np * Np];
   __shared__ ElemMeta<DIM, EPB> sm;
   __shared__ int sfnb[BND ? EPB : 1][BND ? 2 * DIM : 1];  // face neighbours (boundary codes < 0)
-  R (*sS)[NQ][ND] = reinterpret_cast<R (*)[NQ][ND]>(sbuf);
-  R (*sjump)[NFACE][NQ] = reinterpret_cast<R (*)[NFACE][NQ]>(sbuf + EPB * NQ * ND);
+  R (*sS)[NG][ND] = reinterpret_cast<R (*)[NG][ND]>(sbuf);
+  R (*sjump)[NFACE][NG] = reinterpret_cast<R (*)[NFACE][NG]>(sbuf + EPB * NG * ND);
   R (*sG)[DIM][NVD][ND] = reinterpret_cast<R (*)[DIM][NVD][ND]>(sbuf);
 
   const GasC<R> &g = gas_of<R>(a);
@@ -1293,34 +1259,30 @@ __attribute__((amdgpu_waves_per_eu(GradWaves<R, DIM, P, EPBX, BND, LTE>::value))
   meta_load_normals<DIM, EPB, TPB>(a, ebase_blk, mr);
   double qn[NFR][NQ];
   double Tn[LTE ? NFR : 1];
-  int cn[LTE ? NFR : 1];
 #pragma unroll
   for (int r = 0; r < NFR; ++r) {
     const uint32_t fc = kFaceTable<DIM, P, EPBX>.v[min(tid + r * TPB, NFT - 1)];
     const size_t nbase = (size_t)max(fnb[r], 0) * ND + ((fc >> 8) & 255u);
 #pragma unroll
     for (int c = 0; c < NQ; ++c) qn[r][c] = a.U[c * Ntot + nbase];
-    if constexpr (LTE) {
-      Tn[r] = a.lte.node_T[nbase];
-      cn[r] = a.lte.node_cell[nbase];
-    }
+    if constexpr (LTE) Tn[r] = a.lte.node_T[nbase];
   }
   if (tid < Np * Np) {
     sD[tid] = R(bD);
     sDh[tid] = R(bDh);
   }
 
-  // entropy variables of the element's nodes (EOS.hpp:206-234)
+  // variables of the element's nodes (EOS.hpp:206-234)
   meta_store<DIM, EPB, TPB>(mr, sm);
   R q[NQ];
 #pragma unroll
   for (int c = 0; c < NQ; ++c) q[c] = R(q64[c]);
   if (valid) {
-    R Sv[NQ];
-    if constexpr (LTE) lte::entropy_state<DIM>(a.lte, q, R(Town), cown, Sv);
-    else entropy_state<R, DIM>(g, q, Sv);
+    R Sv[NG];
+    if constexpr (LTE) lte::viscous_variables<DIM>(q, R(Town), Sv);
+    else viscous_variables<R, DIM>(g, q, Sv);
 #pragma unroll
-    for (int c = 0; c < NQ; ++c) sS[el][c][node] = Sv[c];
+    for (int c = 0; c < NG; ++c) sS[el][c][node] = Sv[c];
   }
   lds_sync();
 
@@ -1337,24 +1299,24 @@ __attribute__((amdgpu_waves_per_eu(GradWaves<R, DIM, P, EPBX, BND, LTE>::value))
       const int s = (int)(fc >> 28) & 1;
       const int on = (int)(fc & 255u);
       if (!BND || fnb[r] >= 0) {
-        R qr[NQ], Sn[NQ];
+        R qr[NQ], Sn[NG];
 #pragma unroll
         for (int c = 0; c < NQ; ++c) qr[c] = R(qn[r][c]);
-        if constexpr (LTE) lte::entropy_state<DIM>(a.lte, qr, R(Tn[LTE ? r : 0]), cn[LTE ? r : 0], Sn);
-        else entropy_state<R, DIM>(g, qr, Sn);
+        if constexpr (LTE) lte::viscous_variables<DIM>(qr, R(Tn[LTE ? r : 0]), Sn);
+        else viscous_variables<R, DIM>(g, qr, Sn);
 #pragma unroll
-        for (int c = 0; c < NQ; ++c) {
+        for (int c = 0; c < NG; ++c) {
           const R so = sS[pe][c][on];
           sjump[pe][fl][c] = s ? R(0.5) * (Sn[c] - so) : R(0.5) * (so - Sn[c]);
         }
       } else {
         const int b = -(fnb[r] + 1);
-        R So[NQ], jb[NQ];
+        R So[NG], jb[NG];
 #pragma unroll
-        for (int c = 0; c < NQ; ++c) So[c] = sS[pe][c][on];
+        for (int c = 0; c < NG; ++c) So[c] = sS[pe][c][on];
         bc_grad_jump<R, DIM>(g, a.bc_type[b], a.bc_data + (size_t)b * BC_STRIDE, So, jb);
 #pragma unroll
-        for (int c = 0; c < NQ; ++c) sjump[pe][fl][c] = jb[c];
+        for (int c = 0; c < NG; ++c) sjump[pe][fl][c] = jb[c];
       }
     }
   }
@@ -1374,26 +1336,29 @@ __attribute__((amdgpu_waves_per_eu(GradWaves<R, DIM, P, EPBX, BND, LTE>::value))
   for (int c = 0; c < NVD; ++c) hv[c] = R(0);
   constexpr bool MF = GradMfma<R, DIM, P, EPBX>::on && !BND;  // with the boundary code it would cost a wave
   // the line contractions D.S of all directions on the matrix cores (every lane of the wave)
-  float drefm[MF ? 3 : 1][MF ? 5 : 1];
+  float drefm[MF ? 3 : 1][4];
   float opD[4];  // matrix-core operand: row node%4 of D (then of Dhat)
   if constexpr (MF) {
 #pragma unroll
     for (int l = 0; l < 4; ++l) opD[l] = sD[(node & 3) * 4 + l];
-    line_contract_mfma5(reinterpret_cast<const float (*)[64]>(sS[elc]), opD, node, drefm);
+    const float(*F)[64] = reinterpret_cast<const float(*)[64]>(sS[elc]);
+    line_contract_dir<0>(F, opD, node, drefm[0]);
+    line_contract_dir<1>(F, opD, node, drefm[1]);
+    line_contract_dir<2>(F, opD, node, drefm[2]);
   }
   if (valid) {
     // volume gradient (AssembleGradVolumePointKernel): acc[dd] = sum_ref (D.S)_ref adj(ref,dd),
     // one reference direction at a time, in the reference's ref = 0,1,2 order
-    R acc[DIM][NQ];
+    R acc[DIM][NG];
 #pragma unroll MF ? DIM : 1
     for (int dir = 0; dir < DIM; ++dir) {
-      R dref[NQ];
+      R dref[NG];
       if constexpr (MF) {
 #pragma unroll
-        for (int c = 0; c < NQ; ++c) dref[c] = drefm[MF ? dir : 0][MF ? c : 0];
+        for (int c = 0; c < NG; ++c) dref[c] = drefm[MF ? dir : 0][MF ? c : 0];
       } else {
 #pragma unroll
-        for (int c = 0; c < NQ; ++c) dref[c] = R(0);
+        for (int c = 0; c < NG; ++c) dref[c] = R(0);
         const int mi = dir == 0 ? i : (dir == 1 ? j : k);
         const int st = dir == 0 ? 1 : (dir == 1 ? Np : Np * Np);
         const int base = node - mi * st;
@@ -1402,14 +1367,14 @@ __attribute__((amdgpu_waves_per_eu(GradWaves<R, DIM, P, EPBX, BND, LTE>::value))
           const R coef = sD[mi * Np + l];
           const int sn_ = base + l * st;
 #pragma unroll
-          for (int c = 0; c < NQ; ++c) dref[c] += sS[el][c][sn_] * coef;
+          for (int c = 0; c < NG; ++c) dref[c] += sS[el][c][sn_] * coef;
         }
       }
 #pragma unroll
       for (int dd = 0; dd < DIM; ++dd) {
         const R ad = R(sm.adj[el][dir * DIM + dd]);
 #pragma unroll
-        for (int c = 0; c < NQ; ++c) acc[dd][c] = dir == 0 ? dref[c] * ad : acc[dd][c] + dref[c] * ad;
+        for (int c = 0; c < NG; ++c) acc[dd][c] = dir == 0 ? dref[c] * ad : acc[dd][c] + dref[c] * ad;
       }
     }
     using Thermo = std::conditional_t<LTE, lte::ViscNode<DIM, R>, NodeThermo<R, DIM>>;
@@ -1422,16 +1387,16 @@ __attribute__((amdgpu_waves_per_eu(GradWaves<R, DIM, P, EPBX, BND, LTE>::value))
 #pragma unroll
     for (int dd = 0; dd < DIM; ++dd)
 #pragma unroll
-      for (int c = 0; c < NQ; ++c) acc[dd][c] *= invJ;
+      for (int c = 0; c < NG; ++c) acc[dd][c] *= invJ;
 #pragma unroll
     for (int d = 0; d < DIM; ++d) {
       const bool hi = idx[d] == Np - 1;
       const bool on = hi || idx[d] == 0;
       const int f = 2 * d + (hi ? 1 : 0);
       const int row = f * NF + face_index<DIM, Np>(d, i, j, k);
-      R jw[NQ];
+      R jw[NG];
 #pragma unroll
-      for (int c = 0; c < NQ; ++c) {
+      for (int c = 0; c < NG; ++c) {
         const R v = wown * sjump[el][row][c];
         jw[c] = on ? v : R(0);
       }
@@ -1439,13 +1404,14 @@ __attribute__((amdgpu_waves_per_eu(GradWaves<R, DIM, P, EPBX, BND, LTE>::value))
       for (int dd = 0; dd < DIM; ++dd) {
         const R nd = R(sm.nrm[el][f][dd]);
 #pragma unroll
-        for (int c = 0; c < NQ; ++c) acc[dd][c] += jw[c] * nd;
+        for (int c = 0; c < NG; ++c) acc[dd][c] += jw[c] * nd;
       }
     }
-    R dP[DIM][NQ];
+    R dV[DIM][DIM], dT[DIM];
 #pragma unroll
-    for (int dd = 0; dd < DIM; ++dd) grad_entropy_to_grad_prim<R, DIM>(th, q, acc[dd], dP[dd]);
-    viscous_flux<R, DIM>(g, th, dP, vf);
+    for (int dd = 0; dd < DIM; ++dd) viscous_gradients<R, DIM>(g, th, acc[dd], dV[dd], dT[dd]);
+    if constexpr (LTE) viscous_flux<R, DIM>(th.mu, th.kappa, g.mu_bulk, th.u, dV, dT, vf);
+    else viscous_flux<R, DIM>(g.mu, g.kappa, g.mu_bulk, th.u, dV, dT, vf);
 
     // n.Fv at the element's own face points, n the canonical area vector
 #pragma unroll
@@ -1483,7 +1449,7 @@ __attribute__((amdgpu_waves_per_eu(GradWaves<R, DIM, P, EPBX, BND, LTE>::value))
       }
     }
   }
-  lds_sync();  // the entropy/jump buffers are reused below
+  lds_sync();  // the variables and jumps are overwritten below
 
   // contravariant viscous fluxes adj_dir . Fv per node
   if (valid) {
