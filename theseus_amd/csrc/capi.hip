@@ -168,7 +168,10 @@ static void derivative_ops(int p, const std::vector<double> &x, const std::vecto
   b.Dhat[(Np - 1) * Np + Np - 1] -= 1.0 / w[Np - 1];
   b.Dhat2[0] += 1.0 / w[0];
   b.Dhat2[(Np - 1) * Np + Np - 1] -= 1.0 / w[Np - 1];
-  for (int i = 0; i < Np; ++i) b.w[i] = w[i];
+  for (int i = 0; i < Np; ++i) {
+    b.w[i] = w[i];
+    b.iw[i] = 1.0 / w[i];
+  }
 }
 
 // Inverse of the 1-D Legendre Vandermonde V(i,a) = P_a(2 x_i - 1) on the
@@ -458,6 +461,22 @@ static int fail(int code, const std::string &msg) {
     if (_e != hipSuccess) return fail(THESEUS_ERR_DEVICE, std::string(#expr ": ") + hipGetErrorString(_e)); \
   } while (0)
 
+// The sigmoid argument beyond which the blending coefficient, 1/(1 + exp(x)),
+// is certainly below alpha_min and therefore cut to 0.
+static double alpha_cut(double alpha_min) {
+  return alpha_min > 0 && alpha_min < 1 ? std::log(1.0 / alpha_min - 1.0) + 1e-9 : HUGE_VAL;
+}
+
+// Does the fused kernel run in its line form (k_rhs_line) on ne elements?
+// Where it is built, on enough waves to fill the chip (line_min_waves), and
+// where a field of Ntot nodes and a row of n.Fv at ngf face points can be
+// addressed with 32-bit byte offsets.
+static bool line_form(const FluxKernels *fk, bool ns, int ne, long long Ntot, long long ngf) {
+  if (!fk || !(ns ? fk->ns_line : fk->euler_line)) return false;
+  const int waves = (ne + fk->line_epw - 1) / fk->line_epw;
+  return waves >= (ns ? fk->ns_line_min : fk->euler_line_min) && Ntot * 8 < (1LL << 32) && ngf * 8 < (1LL << 32);
+}
+
 struct theseus_rhs {
   theseus_case_desc d;
   int Np, ndof, nfp, neq;
@@ -480,6 +499,7 @@ struct theseus_rhs {
   GasC<double> gas;
   GasC<float> gas32;
   int pm = 0;  // kernel variant: 0 FP64, 1 FP32 flux arithmetic
+  bool line = false;  // the fused kernel's line form (k_rhs_line)
   double adv_scale, diff_scale, surf_scale;
   double *d_J = nullptr, *d_adj = nullptr;
   int *d_nbr = nullptr;
@@ -529,6 +549,7 @@ struct theseus_rhs {
     a.alpha_min = d.alpha_min;
     a.sharp = 9.21024;                                                 // RHSOperator.hpp:33
     a.thresh = 0.5 * std::pow(10.0, -1.8 * std::pow(d.order, 0.25));  // RHSOperator.hpp:53
+    a.alpha_cut = alpha_cut(d.alpha_min);
     a.J = d_J;
     a.adj = d_adj;
     a.nbr = d_nbr;
@@ -584,11 +605,15 @@ static int enqueue_rhs(theseus_rhs *h, RHSArgs a, hipStream_t s) {
       timed(h, 1, s, [&] { h->lk->nodes(a, nb, s); });
       timed(h, 0, s, [&] { h->lk->rhs[h->lfx][h->pm](a, nb, s); });
     }
-  } else if (h->d.flow_model == THESEUS_FLOW_NAVIER_STOKES) {
-    timed(h, 1, s, [&] { h->sk->ns_grad[h->pm][h->has_boundary](a, nb, s); });
-    timed(h, 0, s, [&] { h->fk->ns[h->pm][h->has_boundary](a, nb, s); });
   } else {
-    timed(h, 0, s, [&] { h->fk->euler[h->pm][h->has_boundary](a, nb, s); });
+    const bool ns = h->d.flow_model == THESEUS_FLOW_NAVIER_STOKES;
+    if (ns) timed(h, 1, s, [&] { h->sk->ns_grad[h->pm][h->has_boundary](a, nb, s); });
+    if (h->line) {
+      const int nl = (h->d.num_elements + h->fk->line_epw - 1) / h->fk->line_epw;
+      timed(h, 0, s, [&] { (ns ? h->fk->ns_line : h->fk->euler_line)(a, nl, s); });
+    } else {
+      timed(h, 0, s, [&] { (ns ? h->fk->ns : h->fk->euler)[h->pm][h->has_boundary](a, nb, s); });
+    }
   }
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return fail(THESEUS_ERR_DEVICE, std::string("kernel launch: ") + hipGetErrorString(e));
@@ -915,6 +940,8 @@ static int create_impl(const theseus_case_desc *desc, const theseus_lte_table *l
   h->neq = dim + 2;
   h->Ntot = (long long)ne * h->ndof;
   h->has_boundary = has_boundary;
+  h->line = !has_boundary && d.precision == THESEUS_PRECISION_FP64 &&
+            line_form(fk, d.flow_model == THESEUS_FLOW_NAVIER_STOKES, ne, h->Ntot, (long long)ne * 2 * dim * h->nfp);
   std::vector<double> x, w;
   gll01(d.order, x, w);
   derivative_ops(d.order, x, w, h->basis);
@@ -1694,6 +1721,7 @@ struct theseus_pool {
     a.alpha_min = cd.alpha_min;
     a.sharp = 9.21024;
     a.thresh = 0.5 * std::pow(10.0, -1.8 * std::pow(cd.order, 0.25));
+    a.alpha_cut = alpha_cut(cd.alpha_min);
     a.J = d_J;
     a.adj = d_adj;
     a.nbr = d_nbr;

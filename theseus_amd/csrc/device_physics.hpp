@@ -99,9 +99,9 @@ struct LogMeanEps<float> {
 template <typename R>
 using LogMean = LogMeanPair<R>;
 
-template <typename R, bool NEED_LM, bool NEED_INV>
+template <typename R, bool NEED_LM, bool NEED_INV, bool SERIES = false>
 __device__ __forceinline__ LogMean<R> log_mean2(R x, R y) {
-  return log_mean_pair<R, NEED_LM, NEED_INV>(x, y);
+  return log_mean_pair<R, NEED_LM, NEED_INV, SERIES>(x, y);
 }
 
 // Logarithmic mean in the reference's exact formulation (kept for the
@@ -159,11 +159,11 @@ __device__ __forceinline__ R chandrashekar_p_mom(const Pt<R, DIM> &a, const Pt<R
 }
 
 // ChandrashekarFlux.hpp:20-89
-template <typename R, int DIM>
+template <typename R, int DIM, bool SERIES = false>
 __device__ __forceinline__ void vol_chandrashekar(const GasC<R> &g, const Pt<R, DIM> &a, const Pt<R, DIM> &b,
                                                   const R *met, R *F) {
   const R rho1 = a.q[0], rho2 = b.q[0];
-  const LogMean<R> lr = log_mean2<R, true, true>(rho1, rho2);
+  const LogMean<R> lr = log_mean2<R, true, true, SERIES>(rho1, rho2);
   const R rho_ln = lr.lm;
   R mom_hat[DIM];
   R h_hat = R(0), vn = R(0);
@@ -177,7 +177,7 @@ __device__ __forceinline__ void vol_chandrashekar(const GasC<R> &g, const Pt<R, 
   }
   const R beta1 = R(0.5) * rho1 / a.p;
   const R beta2 = R(0.5) * rho2 / b.p;
-  const R inv_beta_ln = log_mean2<R, false, true>(beta1, beta2).inv;
+  const R inv_beta_ln = log_mean2<R, false, true, SERIES>(beta1, beta2).inv;
   const R p_hat = R(0.5) * (rho1 + rho2) / (beta1 + beta2);
   const R gm1_av_inv = g.gammaM1Inverse;  // 2/(gamma1 + gamma2 - 2) with one gamma
   h_hat += R(0.5) * inv_beta_ln * gm1_av_inv + p_hat * lr.inv;
@@ -189,11 +189,11 @@ __device__ __forceinline__ void vol_chandrashekar(const GasC<R> &g, const Pt<R, 
 }
 
 // RanochaFlux.hpp:20-79
-template <typename R, int DIM>
+template <typename R, int DIM, bool SERIES = false>
 __device__ __forceinline__ void vol_ranocha(const GasC<R> &g, const Pt<R, DIM> &a, const Pt<R, DIM> &b, const R *met,
                                             R *F) {
   const R rho1 = a.q[0], rho2 = b.q[0];
-  const R rho_ln = log_mean2<R, true, false>(rho1, rho2).lm;
+  const R rho_ln = log_mean2<R, true, false, SERIES>(rho1, rho2).lm;
   const R p1 = a.p, p2 = b.p;
   const R pdbar = R(0.5) * (a.pd + b.pd);
   R vbar[DIM], ppm[DIM];
@@ -206,7 +206,7 @@ __device__ __forceinline__ void vol_ranocha(const GasC<R> &g, const Pt<R, DIM> &
     ke_flux += R(0.5) * (v1 * v2);
     ppm[d] = R(0.5) * (p1 * v2 + p2 * v1);
   }
-  const R inv_beta_ln = (p1 * p2) * log_mean2<R, false, true>(rho1 * p2, rho2 * p1).inv;
+  const R inv_beta_ln = (p1 * p2) * log_mean2<R, false, true, SERIES>(rho1 * p2, rho2 * p1).inv;
   const R inv_gm1 = g.gammaM1Inverse;
   const R ie_flux = inv_beta_ln * inv_gm1;
   R fe = R(0);
@@ -643,13 +643,14 @@ __device__ __forceinline__ void face_llf_signed(const GasC<R> &g, const Pt<R, DI
   }
 }
 
-// Compile-time flux selection (ids of include/theseus_rhs.h)
-template <int VOL, typename R, int DIM>
+// Compile-time flux selection (ids of include/theseus_rhs.h).  SERIES: the
+// pair's logarithmic means are known to be in log_mean_pair's first branch.
+template <int VOL, typename R, int DIM, bool SERIES = false>
 __device__ __forceinline__ void volume_flux(const GasC<R> &g, const Pt<R, DIM> &a, const Pt<R, DIM> &b, const R *met,
                                             R *F) {
   if constexpr (VOL == 0) vol_central<R, DIM>(g, a, b, met, F);
-  else if constexpr (VOL == 1) vol_chandrashekar<R, DIM>(g, a, b, met, F);
-  else if constexpr (VOL == 2) vol_ranocha<R, DIM>(g, a, b, met, F);
+  else if constexpr (VOL == 1) vol_chandrashekar<R, DIM, SERIES>(g, a, b, met, F);
+  else if constexpr (VOL == 2) vol_ranocha<R, DIM, SERIES>(g, a, b, met, F);
   else vol_pirozzoli<R, DIM>(g, a, b, met, F);
 }
 

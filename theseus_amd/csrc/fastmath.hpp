@@ -108,13 +108,14 @@ struct LogMeanPair {
   R lm, inv;
 };
 
-template <typename R, bool NEED_LM, bool NEED_INV>
+// SERIES: the caller knows the pair to be in the first branch.
+template <typename R, bool NEED_LM, bool NEED_INV, bool SERIES = false>
 __host__ __device__ __forceinline__ LogMeanPair<R> log_mean_pair(R x, R y) {
   constexpr bool F64 = sizeof(R) == sizeof(double);
   LogMeanPair<R> r{R(0), R(0)};
   const R s = x + y;
   const R d = y - x;
-  if (d * d < R(F64 ? 1e-4 : 1e-2) * (s * s)) {
+  if (SERIES || d * d < R(F64 ? 1e-4 : 1e-2) * (s * s)) {
     const R rs = recip_refined<R>(s);
     const R t = d * rs;
     const R u = t * t;

@@ -7,6 +7,7 @@
 #include <hip/hip_runtime.h>
 
 #include "rhs_kernels.hpp"
+#include "rhs_line.hpp"
 #include "rhs_lte.hpp"
 
 namespace thx {
@@ -21,6 +22,11 @@ using MeasLaunch = void (*)(const MeasArgs &, int nblocks, hipStream_t);
 struct FluxKernels {
   RHSLaunch euler[2][2] = {};  // fused volume + face
   RHSLaunch ns[2][2] = {};     // Navier-Stokes pass 2
+  // the FP64 line form (k_rhs_line) on meshes without boundary faces, and the
+  // fewest workgroups (waves of line_epw elements) it is used from; null where it is not built
+  RHSLaunch euler_line = nullptr, ns_line = nullptr;
+  int euler_line_min = 0, ns_line_min = 0;
+  int line_epw = 0;
 };
 
 struct ShapeKernels {
@@ -89,10 +95,55 @@ void launch_measures(const MeasArgs &a, int nb, hipStream_t s) {
   hipLaunchKernelGGL((k_measures<DIM, P>), dim3(nb), dim3(Shape<DIM, P>::TPB), 0, s, a);
 }
 
+// From how many waves on the line form (k_rhs_line) is the faster one, 0 where
+// it is not built.  It issues 0.4 to 0.6 of the node form's instructions but
+// runs Np nodes in each lane's chain, so it needs waves to hide latency: one
+// per SIMD (1024 waves) is about where it begins to win.  Ratio of the times,
+// node / line form, of a whole evaluation at 512, 1024, 2048 and 4096 waves:
+//   FP64 3-D p = 3  Ranocha/LLF Euler 1.32 1.42 1.69 1.53, NS 1.09 1.07 1.22 1.14;
+//                   central/HLL Euler 1.20 1.28 1.55 1.40, NS 1.01 1.02 1.21 1.13;
+//                   Chandrashekar/Roe Euler 1.16 1.54 1.53 1.47, NS 0.96 1.09 1.24 1.16
+//   FP64 3-D p = 2  Ranocha/LLF Euler 1.21 1.46 1.42 1.65, NS 0.94 1.18 0.99 1.16
+//   FP64 2-D p = 3  Ranocha/LLF Euler 1.06 1.22 1.52 1.47, NS 0.98 1.10 1.26 1.20
+// Order 4 in 3-D (two elements in 50 of 64 lanes, five nodes a lane) needs the
+// registers: Ranocha/LLF Euler 1.02 1.15 1.52 1.52, central/LLF 0.99 1.08 1.38
+// 1.31, Ranocha/LLF NS 0.90 1.04 1.19 1.14, but central/HLL NS 0.63 0.78 0.86
+// 0.81 and Chandrashekar's 0.60 0.77 1.03 0.99, where it is left out, as
+// Pirozzoli's is (0.96 1.22 1.20 1.26 at p = 2 Euler, NS 0.68 0.91 0.89 0.86)
+// and Chandrashekar's in 2-D NS at p = 4 (0.65 0.92 0.97 1.07).
+// In the mixed mode, whose node form is shorter and whose line form holds three
+// sets of sums, the ratios at p = 3 were 1.03 1.06 1.33 1.14 for Euler and 0.96
+// 0.98 1.14 1.02 for NS, at p = 4 0.81 0.89 1.15 1.09 and 0.82 0.96 1.10 1.04,
+// and a pool's results would depend on its launch range: FP64 only.
+template <int DIM, int P, int VOL, int SURF>
+constexpr int line_min_waves(bool visc) {
+  if (P < 2 || P > 4 || VOL == 3) return 0;
+  if (DIM == 3 && P == 4) {
+    if (VOL == 1 || (visc && VOL != 2)) return 0;
+    return VOL == 2 && SURF == 5 && !visc ? 1024 : 2048;
+  }
+  if (DIM == 2 && P == 4 && VOL == 1 && visc) return 0;
+  return DIM == 3 && P == 3 && !visc ? 512 : 1024;
+}
+
+template <int DIM, int P, int VOL, int SURF, bool VISC>
+void launch_rhs_line(const RHSArgs &a, int nb, hipStream_t s) {
+  hipLaunchKernelGGL((k_rhs_line<DIM, P, VOL, SURF, VISC>), dim3(nb), dim3(64), 0, s, a);
+}
+
 template <int DIM, int VOL, int SURF, int P>
 struct FluxRegistrar {
   FluxRegistrar() {
     FluxKernels k;
+    if constexpr (line_min_waves<DIM, P, VOL, SURF>(false) > 0) {
+      k.euler_line = &launch_rhs_line<DIM, P, VOL, SURF, false>;
+      k.euler_line_min = line_min_waves<DIM, P, VOL, SURF>(false);
+      k.line_epw = LineShape<DIM, P>::EPW;
+    }
+    if constexpr (line_min_waves<DIM, P, VOL, SURF>(true) > 0) {
+      k.ns_line = &launch_rhs_line<DIM, P, VOL, SURF, true>;
+      k.ns_line_min = line_min_waves<DIM, P, VOL, SURF>(true);
+    }
     k.euler[0][0] = &launch_rhs<double, DIM, P, VOL, SURF, false>;
     k.ns[0][0] = &launch_rhs<double, DIM, P, VOL, SURF, true>;
     k.euler[1][0] = &launch_rhs<float, DIM, P, VOL, SURF, false>;

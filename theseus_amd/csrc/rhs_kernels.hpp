@@ -53,6 +53,7 @@ struct BasisArgs {
   double Dhat[MAXNP * MAXNP];   // D + (1/w0) e0 e0^T - (1/wN) eN eN^T
   double Dhat2[MAXNP * MAXNP];  // 2D with the same corner corrections
   double w[MAXNP];              // GLL weights on [0,1]
+  double iw[MAXNP];             // their reciprocals
   double Vinv[MAXNP * MAXNP];   // inverse 1-D Legendre Vandermonde: mode a = sum_i Vinv[a*Np+i] u_i
 };
 
@@ -73,6 +74,7 @@ struct RHSCore {
   int ne;
   int blending;
   double alpha_max, alpha_min, sharp, thresh;
+  double alpha_cut;     // ln(1/alpha_min - 1) and a margin for rounding (infinite if alpha_min <= 0)
   const double *J;      // [ne]
   const double *adj;    // [ne][DIM][DIM]
   const int *nbr;       // [ne][2*DIM]; -(b+1) on a face of boundary b
@@ -95,6 +97,15 @@ struct RHSCore {
 struct RHSArgs : RHSCore {
   BasisArgs basis;
 };
+
+// What a kernel writes for a node whose rate of change is r: the rate, a
+// forward Euler stage from the stage state q, or the SSP-RK3 combination with
+// the base state x.  Rounded the same way wherever it is inlined.
+__device__ __forceinline__ double stage_value(const RHSCore &a, double dt, double x, double q, double r) {
+  if (a.mode == 0) return r;
+  const double u = fma(dt, r, q);
+  return a.mode == 1 ? u : fma(a.cx, x, a.cy * u);
+}
 
 template <typename R>
 __device__ __forceinline__ const GasC<R> &gas_of(const RHSCore &a);
@@ -140,6 +151,27 @@ __device__ __forceinline__ int logical_block(int remap) {
   const int nb = gridDim.x, b = blockIdx.x;
   if (remap && (nb & 7) == 0) return (b & 7) * (nb >> 3) + (b >> 3);
   return b;
+}
+
+// The blending coefficient from the sums of the squared modes: all, those of
+// degree <= p-1 and those of degree <= p-2 in every direction.
+__device__ __forceinline__ double alpha_of_modes(const RHSCore &a, double mm, double m1m1, double m2m2) {
+  const double eps = 1.0e-30;
+  double val = 0.0;
+  if (mm > eps) {
+    val = 1.0 - m1m1 / mm;
+    if (m1m1 > eps) val = fmax(val, 1.0 - m2m2 / m1m1);
+    else val = 1.0;
+  }
+  const double eta = fmin(fmax(val, 0.0), 1.0);
+  // the sigmoid's argument; beyond alpha_cut the sigmoid is below alpha_min
+  // and the coefficient 0, as in almost every element, without the exponential
+  const double x = -a.sharp * (eta - a.thresh) / a.thresh;
+  if (x > a.alpha_cut) return fmin(0.0, a.alpha_max);
+  double al = 1.0 / (1.0 + exp(x));
+  if (al < a.alpha_min) al = 0.0;
+  else if (al > (1.0 - a.alpha_min)) al = 1.0;
+  return fmin(al, a.alpha_max);
 }
 
 // Persson-Peraire indicator of one element (RHSOperator_impl.hpp:355-527):
@@ -224,18 +256,7 @@ __device__ __forceinline__ double blending_alpha(const RHSCore &a, double *buf, 
     m1m1 = red[NP2];
     m2m2 = red[2 * NP2];
   }
-  const double eps = 1.0e-30;
-  double val = 0.0;
-  if (mm > eps) {
-    val = 1.0 - m1m1 / mm;
-    if (m1m1 > eps) val = fmax(val, 1.0 - m2m2 / m1m1);
-    else val = 1.0;
-  }
-  const double eta = fmin(fmax(val, 0.0), 1.0);
-  double al = 1.0 / (1.0 + exp(-a.sharp * (eta - a.thresh) / a.thresh));
-  if (al < a.alpha_min) al = 0.0;
-  else if (al > (1.0 - a.alpha_min)) al = 1.0;
-  return fmin(al, a.alpha_max);
+  return alpha_of_modes(a, mm, m1m1, m2m2);
 }
 
 // ---------------------------------------------------------------------------
@@ -1027,11 +1048,7 @@ __device__ __forceinline__ void rhs_body(const RHSCore &a, const BasisArgs &B, c
       double qo;
       if constexpr (FP64) qo = sq[el][q][SX::at(node)];
       else qo = q64[q];
-      double o;
-      if (a.mode == 0) o = r;
-      else if (a.mode == 1) o = qo + dt * r;
-      else o = a.cx * xb[q] + a.cy * (qo + dt * r);
-      a.out[q * Ntot + ebase] = o;
+      a.out[q * Ntot + ebase] = stage_value(a, dt, xb[q], qo, r);
     }
   }
 }
