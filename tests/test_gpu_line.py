@@ -1,6 +1,6 @@
-"""The fused kernel's line form (meshes without boundary faces, enough
-elements to fill the chip) against the CPU oracle, at the element counts from
-which it is used (odd counts: the last wave is partly filled), on states that
+"""The line forms of the fused kernel and the gradient pass (FP64, meshes
+without boundary faces, enough elements to fill the chip) against the CPU
+oracle, at the element counts from which they are used (odd counts: the last wave is partly filled), on states that
 take each branch of the logarithmic means, with and without blended elements.
 The bound is that of the other FP64 RHS tests, relative L2 <= 1e-12."""
 import numpy as np
@@ -35,6 +35,7 @@ def _state(mesh, order, gamma, noise):
     (3, (13, 13, 13), 3, "ranocha_llf", False), (3, (13, 13, 13), 3, "hll", False),           # 550 waves of 4
     (3, (17, 15, 17), 3, "ranocha_llf", True), (3, (17, 15, 17), 3, "chandrashekar_roe", True),
     (3, (13, 13, 13), 4, "ranocha_llf", False), (3, (17, 15, 17), 4, "ranocha_llf", True),    # waves of 2
+    (3, (13, 13, 13), 3, "hll", True), (2, (107, 107), 2, "hll", True), (2, (91, 91), 3, "llf", True),  # the gradient pass alone
     (2, (147, 147), 2, "llf", False), (2, (129, 128), 3, "ranocha_llf", False),
     (2, (111, 111), 4, "ranocha", True),
 ])

@@ -467,14 +467,37 @@ static double alpha_cut(double alpha_min) {
   return alpha_min > 0 && alpha_min < 1 ? std::log(1.0 / alpha_min - 1.0) + 1e-9 : HUGE_VAL;
 }
 
-// Does the fused kernel run in its line form (k_rhs_line) on ne elements?
-// Where it is built, on enough waves to fill the chip (line_min_waves), and
-// where a field of Ntot nodes and a row of n.Fv at ngf face points can be
-// addressed with 32-bit byte offsets.
-static bool line_form(const FluxKernels *fk, bool ns, int ne, long long Ntot, long long ngf) {
+// Can the line forms (k_rhs_line, k_ns_grad_line) address ne elements' fields
+// and n.Fv rows with 32-bit byte offsets?
+static bool line_offsets(int ne, int ndof, int dim, int nfp) {
+  return (long long)ne * std::max(ndof, 2 * dim * nfp) * 8 < (1LL << 32);
+}
+
+// Does the fused kernel run in its line form on ne elements?  Where it is
+// built, on enough waves to fill the chip (line_min_waves).
+static bool line_form(const FluxKernels *fk, bool ns, int ne) {
   if (!fk || !(ns ? fk->ns_line : fk->euler_line)) return false;
-  const int waves = (ne + fk->line_epw - 1) / fk->line_epw;
-  return waves >= (ns ? fk->ns_line_min : fk->euler_line_min) && Ntot * 8 < (1LL << 32) && ngf * 8 < (1LL << 32);
+  return (ne + fk->line_epw - 1) / fk->line_epw >= (ns ? fk->ns_line_min : fk->euler_line_min);
+}
+
+// Does the gradient pass?  Where it is built, on enough waves
+// (grad_line_min_waves), and where every element's face area vectors (adj
+// rows) are its neighbours' to rounding, as the line form takes an element's own.
+static bool grad_line_form(const ShapeKernels *sk, const theseus_case_desc &d) {
+  if (!sk->ns_grad_line || (d.num_elements + sk->line_epw - 1) / sk->line_epw < sk->ns_grad_line_min) return false;
+  const int dim = d.dim;
+  for (long long e = 0; e < d.num_elements; ++e)
+    for (int k = 0; k < dim; ++k) {
+      const double *own = d.elem_adj + (e * dim + k) * dim;
+      const double *low = d.elem_adj + ((long long)d.face_neighbor[e * 2 * dim + 2 * k] * dim + k) * dim;
+      double diff = 0.0, size = 0.0;
+      for (int c = 0; c < dim; ++c) {
+        diff += std::fabs(own[c] - low[c]);
+        size += std::fabs(own[c]);
+      }
+      if (!(diff <= 1e-13 * size)) return false;
+    }
+  return true;
 }
 
 struct theseus_rhs {
@@ -499,7 +522,8 @@ struct theseus_rhs {
   GasC<double> gas;
   GasC<float> gas32;
   int pm = 0;  // kernel variant: 0 FP64, 1 FP32 flux arithmetic
-  bool line = false;  // the fused kernel's line form (k_rhs_line)
+  bool line = false;       // the fused kernel's line form (k_rhs_line)
+  bool grad_line = false;  // the gradient pass's line form (k_ns_grad_line)
   double adv_scale, diff_scale, surf_scale;
   double *d_J = nullptr, *d_adj = nullptr;
   int *d_nbr = nullptr;
@@ -607,7 +631,12 @@ static int enqueue_rhs(theseus_rhs *h, RHSArgs a, hipStream_t s) {
     }
   } else {
     const bool ns = h->d.flow_model == THESEUS_FLOW_NAVIER_STOKES;
-    if (ns) timed(h, 1, s, [&] { h->sk->ns_grad[h->pm][h->has_boundary](a, nb, s); });
+    if (ns && h->grad_line) {
+      const int nl = (h->d.num_elements + h->sk->line_epw - 1) / h->sk->line_epw;
+      timed(h, 1, s, [&] { h->sk->ns_grad_line(a, nl, s); });
+    } else if (ns) {
+      timed(h, 1, s, [&] { h->sk->ns_grad[h->pm][h->has_boundary](a, nb, s); });
+    }
     if (h->line) {
       const int nl = (h->d.num_elements + h->fk->line_epw - 1) / h->fk->line_epw;
       timed(h, 0, s, [&] { (ns ? h->fk->ns_line : h->fk->euler_line)(a, nl, s); });
@@ -940,14 +969,17 @@ static int create_impl(const theseus_case_desc *desc, const theseus_lte_table *l
   h->neq = dim + 2;
   h->Ntot = (long long)ne * h->ndof;
   h->has_boundary = has_boundary;
-  h->line = !has_boundary && d.precision == THESEUS_PRECISION_FP64 &&
-            line_form(fk, d.flow_model == THESEUS_FLOW_NAVIER_STOKES, ne, h->Ntot, (long long)ne * 2 * dim * h->nfp);
   std::vector<double> x, w;
   gll01(d.order, x, w);
   derivative_ops(d.order, x, w, h->basis);
   legendre_vandermonde_inverse(d.order, x, h->basis.Vinv);
   init_gas(d, h->gas, h->gas32);
   h->pm = d.precision == THESEUS_PRECISION_MIXED ? 1 : 0;
+  if (!has_boundary && !lk && h->pm == 0 && line_offsets(ne, h->ndof, dim, h->nfp)) {
+    const bool ns = d.flow_model == THESEUS_FLOW_NAVIER_STOKES;
+    h->line = line_form(fk, ns, ne);
+    h->grad_line = ns && grad_line_form(sk, d);
+  }
   h->adv_scale = advection_scale(d.order);
   h->diff_scale = diffusion_scale(d.order);
   h->surf_scale = h->adv_scale / (1.0 / w[0]);

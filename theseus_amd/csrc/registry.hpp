@@ -7,6 +7,7 @@
 #include <hip/hip_runtime.h>
 
 #include "rhs_kernels.hpp"
+#include "grad_line.hpp"
 #include "rhs_line.hpp"
 #include "rhs_lte.hpp"
 
@@ -31,6 +32,11 @@ struct FluxKernels {
 
 struct ShapeKernels {
   RHSLaunch ns_grad[2][2] = {};  // Navier-Stokes pass 1
+  // its FP64 line form (k_ns_grad_line) on meshes without boundary faces, and the fewest
+  // workgroups (waves of line_epw elements) it is used from; null where it is not built
+  RHSLaunch ns_grad_line = nullptr;
+  int ns_grad_line_min = 0;
+  int line_epw = 0;
   StabLaunch stability = nullptr;
   MeasLaunch measures = nullptr;
   int tpb = 0, epb = 0;
@@ -84,6 +90,10 @@ void launch_rhs(const RHSArgs &a, int nb, hipStream_t s) {
 template <typename R, int DIM, int P, bool BND = false>
 void launch_ns_grad(const RHSArgs &a, int nb, hipStream_t s) {
   hipLaunchKernelGGL((k_ns_grad<R, DIM, P, 0, BND>), dim3(nb), dim3(Shape<DIM, P>::TPB), 0, s, a);
+}
+template <int DIM, int P>
+void launch_ns_grad_line(const RHSArgs &a, int nb, hipStream_t s) {
+  hipLaunchKernelGGL((k_ns_grad_line<DIM, P>), dim3(nb), dim3(64), 0, s, a);
 }
 template <int DIM, int P>
 void launch_stability(const StabArgs &a, int nb, hipStream_t s) {
@@ -256,6 +266,16 @@ struct LteFluxRegistrar {
   }
 };
 
+// From how many waves on the gradient pass's line form (k_ns_grad_line) is the
+// faster one, 0 where it is not built.  Ratio of the times, node / line form, of
+// a whole Navier-Stokes evaluation (Ranocha/LLF) at 256, 512, 1024, 2048 and
+// 4096 waves:
+//   3-D  p = 2 1.01 1.06 1.10 1.10 1.07, p = 3 1.03 1.06 1.17 1.16 1.11,
+//        p = 4 0.96 0.99 1.02 1.09 1.16
+//   2-D  p = 2 1.04 1.03 1.07 1.03 1.07, p = 3 1.06 1.03 1.07 1.09 1.08,
+//        p = 4 0.97 0.98 1.04 1.05 1.13
+constexpr int grad_line_min_waves(int p) { return p < 2 || p > 4 ? 0 : (p == 4 ? 1024 : 512); }
+
 template <int DIM, int P>
 struct ShapeRegistrar {
   ShapeRegistrar() {
@@ -264,6 +284,11 @@ struct ShapeRegistrar {
     k.ns_grad[1][0] = &launch_ns_grad<float, DIM, P>;
     k.ns_grad[0][1] = &launch_ns_grad<double, DIM, P, true>;
     k.ns_grad[1][1] = &launch_ns_grad<float, DIM, P, true>;
+    if constexpr (grad_line_min_waves(P) > 0) {
+      k.ns_grad_line = &launch_ns_grad_line<DIM, P>;
+      k.ns_grad_line_min = grad_line_min_waves(P);
+      k.line_epw = LineShape<DIM, P>::EPW;
+    }
     k.stability = &launch_stability<DIM, P>;
     k.measures = &launch_measures<DIM, P>;
     k.tpb = Shape<DIM, P>::TPB;
