@@ -109,19 +109,23 @@ void launch_measures(const MeasArgs &a, int nb, hipStream_t s) {
 // it is not built.  It issues 0.4 to 0.6 of the node form's instructions but
 // runs Np nodes in each lane's chain, so it needs waves to hide latency: one
 // per SIMD (1024 waves) is about where it begins to win.  Ratio of the times,
-// node / line form, of a whole evaluation at 512, 1024, 2048 and 4096 waves:
-//   FP64 3-D p = 3  Ranocha/LLF Euler 1.32 1.42 1.69 1.53, NS 1.09 1.07 1.22 1.14;
-//                   central/HLL Euler 1.20 1.28 1.55 1.40, NS 1.01 1.02 1.21 1.13;
-//                   Chandrashekar/Roe Euler 1.16 1.54 1.53 1.47, NS 0.96 1.09 1.24 1.16
-//   FP64 3-D p = 2  Ranocha/LLF Euler 1.21 1.46 1.42 1.65, NS 0.94 1.18 0.99 1.16
-//   FP64 2-D p = 3  Ranocha/LLF Euler 1.06 1.22 1.52 1.47, NS 0.98 1.10 1.26 1.20
+// node / line form, of a whole evaluation (with NS also of the gradient pass)
+// at 512, 1024, 2048 and 4096 waves:
+//   3-D p = 3  Ranocha/LLF Euler 1.27 1.46 1.81 1.75, NS 1.15 1.25 1.44 1.42;
+//              central/HLL Euler 1.13 1.28 1.58 1.52, NS 0.95 0.99 1.19 1.21;
+//              Chandrashekar/Roe Euler 1.10 1.52 1.49 1.44, NS 0.90 1.10 1.27 1.17
+//   3-D p = 2  Ranocha/LLF Euler 1.14 1.49 1.64 1.56, NS 1.12 1.29 1.35 1.21;
+//              Chandrashekar/Roe Euler 1.06 1.49 1.49 1.38, NS 1.05 1.32 1.38 1.23
+//   2-D p = 3  Ranocha/LLF Euler 1.01 1.19 1.44 1.44, NS 0.97 1.12 1.25 1.29;
+//              Chandrashekar/Roe Euler 0.83 1.04 1.26 1.29, NS 0.91 1.04 1.21 1.21
 // Order 4 in 3-D (two elements in 50 of 64 lanes, five nodes a lane) needs the
-// registers: Ranocha/LLF Euler 1.02 1.15 1.52 1.52, central/LLF 0.99 1.08 1.38
-// 1.31, Ranocha/LLF NS 0.90 1.04 1.19 1.14, but central/HLL NS 0.63 0.78 0.86
-// 0.81 and Chandrashekar's 0.60 0.77 1.03 0.99, where it is left out, as
-// Pirozzoli's is (0.96 1.22 1.20 1.26 at p = 2 Euler, NS 0.68 0.91 0.89 0.86)
-// and Chandrashekar's in 2-D NS at p = 4 (0.65 0.92 0.97 1.07).
-// In the mixed mode, whose node form is shorter and whose line form holds three
+// registers: Ranocha/LLF Euler 1.04 1.26 1.62 1.57, NS 0.91 1.04 1.31 1.30,
+// Ranocha/Ranocha NS 0.76 0.93 1.17 1.16, central/LLF NS 0.79 0.95 1.14 1.06,
+// central/HLL Euler 0.78 0.89 1.11 1.02, but NS 0.61 0.75 0.93 0.88 and
+// Chandrashekar's Euler 0.62 0.78 1.02 0.96, where it is left out, as it is for
+// Chandrashekar's 2-D NS at p = 4 (0.68 0.91 0.97 1.22) and Pirozzoli's (3-D
+// p = 3 Euler 0.83 0.96 1.06 1.02, NS 0.60 0.76 0.89 0.84).
+// In the mixed mode, whose node form is shorter and whose line form held three
 // sets of sums, the ratios at p = 3 were 1.03 1.06 1.33 1.14 for Euler and 0.96
 // 0.98 1.14 1.02 for NS, at p = 4 0.81 0.89 1.15 1.09 and 0.82 0.96 1.10 1.04,
 // and a pool's results would depend on its launch range: FP64 only.
@@ -129,11 +133,11 @@ template <int DIM, int P, int VOL, int SURF>
 constexpr int line_min_waves(bool visc) {
   if (P < 2 || P > 4 || VOL == 3) return 0;
   if (DIM == 3 && P == 4) {
-    if (VOL == 1 || (visc && VOL != 2)) return 0;
-    return VOL == 2 && SURF == 5 && !visc ? 1024 : 2048;
+    if (VOL == 1 || (VOL == 0 && SURF != 5 && visc)) return 0;
+    return VOL == 2 && (!visc || SURF == 5) ? 1024 : 2048;
   }
   if (DIM == 2 && P == 4 && VOL == 1 && visc) return 0;
-  return DIM == 3 && P == 3 && !visc ? 512 : 1024;
+  return DIM == 3 && (SURF == 5 || (P == 3 && !visc)) ? 512 : 1024;
 }
 
 template <int DIM, int P, int VOL, int SURF, bool VISC>

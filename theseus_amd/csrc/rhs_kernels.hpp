@@ -146,12 +146,17 @@ __device__ __forceinline__ void lds_sync() { asm volatile("s_waitcnt lgkmcnt(0)\
 
 // XCD-aware block order: the 8 XCDs each receive a contiguous range of
 // elements so that face neighbours share an L2 (hardware dispatches
-// workgroups round-robin over the XCDs).  `remap` = 0 keeps the launch order.
-__device__ __forceinline__ int logical_block(int remap) {
-  const int nb = gridDim.x, b = blockIdx.x;
-  if (remap && (nb & 7) == 0) return (b & 7) * (nb >> 3) + (b >> 3);
-  return b;
+// workgroups round-robin over the XCDs).  Bit kXcdRanges of `order` clear keeps
+// the launch order; bit kReverse runs each XCD's range backwards.
+enum { kXcdRanges = 1, kReverse = 2 };
+__device__ __forceinline__ int block_order(int b, int nb, int order) {
+  if (!(order & kXcdRanges)) return b;
+  const int x = b & 7, q = nb >> 3, r = nb & 7;
+  const int n = q + (x < r ? 1 : 0);  // blocks of XCD x
+  const int i = b >> 3;
+  return x * q + min(x, r) + (order & kReverse ? n - 1 - i : i);
 }
+__device__ __forceinline__ int logical_block(int order) { return block_order(blockIdx.x, gridDim.x, order); }
 
 // The blending coefficient from the sums of the squared modes: all, those of
 // degree <= p-1 and those of degree <= p-2 in every direction.
@@ -1095,22 +1100,19 @@ __attribute__((amdgpu_waves_per_eu(sizeof(R) == sizeof(double) || BND ? 4 : 5)))
     RhsLds<R, 3, 4, 0> p4;
   } lds;
   const int b = blockIdx.x;
-  auto remap = [](int lb, int nb, int remap_on) {
-    return (remap_on && (nb & 7) == 0) ? (lb & 7) * (nb >> 3) + (lb >> 3) : lb;
-  };
   if (b < off0) {
     if (b >= nb0) return;
-    rhs_body<R, 3, 2, VOL, SURF, false, 4, BND>(a2, basis[0], remap(b, nb0, a2.xcd_remap),
+    rhs_body<R, 3, 2, VOL, SURF, false, 4, BND>(a2, basis[0], block_order(b, nb0, a2.xcd_remap),
                                                 RhsLdsRef<R, 3, 2, 4>::of(lds.p2));
   } else if (b < off1) {
     const int lb = b - off0;
     if (lb >= nb1) return;
-    rhs_body<R, 3, 3, VOL, SURF, false, 0, BND>(a3, basis[1], remap(lb, nb1, a3.xcd_remap),
+    rhs_body<R, 3, 3, VOL, SURF, false, 0, BND>(a3, basis[1], block_order(lb, nb1, a3.xcd_remap),
                                                 RhsLdsRef<R, 3, 3, 0>::of(lds.p3));
   } else {
     const int lb = b - off1;
     if (lb >= nb2) return;
-    rhs_body<R, 3, 4, VOL, SURF, false, 0, BND>(a4, basis[2], remap(lb, nb2, a4.xcd_remap),
+    rhs_body<R, 3, 4, VOL, SURF, false, 0, BND>(a4, basis[2], block_order(lb, nb2, a4.xcd_remap),
                                                 RhsLdsRef<R, 3, 4, 0>::of(lds.p4));
   }
 }

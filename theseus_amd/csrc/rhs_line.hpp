@@ -12,12 +12,17 @@
 // element-wise quantity (normals, Jacobian) is loaded by the lanes that use
 // it, and a workgroup is one wave without barriers.
 //
-// Bound by the issue of FP64 arithmetic (4 clocks per wave instruction).  On
-// 32^3 elements, p = 3, Ranocha/LLF with viscous terms, the kernel takes 109 us
-// for the node form's 173 with 20.8 M vector instructions for 52.9 M, at 218
-// registers (two waves a SIMD; three waves spill and are slower); an SSP-RK3
-// step there takes 544 us for 698, on 48^3 1840 for 2360, and an Euler
-// evaluation on 17 x 15 x 13 elements at p = 4 24.2 us for 32.0.
+// The vector memory path (TD busy 80 % of the time) bounds it more than HBM
+// or the FP64 issue (35 %), so own data moves in memory order, 512 consecutive
+// bytes a wave instruction, and changes to lines in LDS, neighbours along x
+// come from the wave's own LDS, and per-element values are loaded by
+// consecutive lanes once.  With a lane loading and storing its x-line's nodes
+// (32 bytes apart) and each element's values in all its lanes, an SSP-RK3 step
+// on 48^3 elements, p = 3, Ranocha/LLF with viscous terms took 1761 us, now
+// 1600; an Euler evaluation on 17 x 15 x 13 elements at p = 4 24.5 us, now 22.3.
+// On 32^3 elements the kernel takes 107 us for the node form's 173, with 21 M
+// vector instructions for 53 M, at 246 registers: two waves a SIMD (three spill
+// and are slower).
 #pragma once
 
 #include "rhs_kernels.hpp"
@@ -212,11 +217,50 @@ __device__ __forceinline__ void line_volume(const GasC<double> &g, const Pt<doub
     }
 }
 
+// What the lanes of a wave share of its elements e0, ..., e0 + nv - 1: loaded
+// by consecutive lanes (a load per lane of the one value its element's lanes
+// all need would occupy the vector memory path as much as a node's), read
+// from LDS.  Elements past the last hold the last one's.
+template <int DIM, int P>
+struct LineMeta {
+  static constexpr int EPW = LineShape<DIM, P>::EPW;
+  double adj[EPW][DIM * DIM];
+  double J[EPW];
+  int nbr[EPW][2 * DIM];
+
+  // one lane's loads, issued before they are stored
+  struct Regs {
+    static constexpr int NA = (EPW * DIM * DIM + 63) / 64, NN = (EPW * 2 * DIM + 63) / 64;
+    double adj[NA], J;
+    int nbr[NN];
+  };
+  __device__ static __forceinline__ Regs load(const RHSCore &a, int e0, int nv, int lane) {
+    Regs r;
+#pragma unroll
+    for (int k = 0; k < Regs::NN; ++k) r.nbr[k] = a.nbr[(size_t)e0 * 2 * DIM + min(lane + 64 * k, nv * 2 * DIM - 1)];
+#pragma unroll
+    for (int k = 0; k < Regs::NA; ++k) r.adj[k] = a.adj[(size_t)e0 * DIM * DIM + min(lane + 64 * k, nv * DIM * DIM - 1)];
+    r.J = a.J[e0 + min(lane, nv - 1)];
+    return r;
+  }
+  __device__ __forceinline__ void store(const Regs &r, int lane) {
+#pragma unroll
+    for (int k = 0; k < Regs::NN; ++k)
+      if (lane + 64 * k < EPW * 2 * DIM) (&nbr[0][0])[lane + 64 * k] = r.nbr[k];
+#pragma unroll
+    for (int k = 0; k < Regs::NA; ++k)
+      if (lane + 64 * k < EPW * DIM * DIM) (&adj[0][0])[lane + 64 * k] = r.adj[k];
+    if (lane < EPW) J[lane] = r.J;
+  }
+};
+
 template <int DIM, int P>
 struct LineLds {
   using S = LineShape<DIM, P>;
   double q[S::NQ][S::EPW * S::NDS];
   double x[S::EPW * S::NDS];  // one field on its way between directions
+  LineMeta<DIM, P> m;
+  double nl[S::EPW][DIM * DIM];  // the adjugate rows of the low-side neighbours
 };
 
 // Moves one value per node from the lines of one direction to those of
@@ -230,6 +274,22 @@ __device__ __forceinline__ void line_move(double *buf, int from, int fstride, in
 #pragma unroll
   for (int m = 0; m < Np; ++m) v[m] = buf[to + m * tstride];
   __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+}
+
+// The running sums' move, one field at a time
+template <int DIM, int P>
+__device__ __forceinline__ void line_move_sums(LineLds<DIM, P> &L, int from, int fstride, int to, int tstride,
+                                               double (*rate)[DIM + 2]) {
+  constexpr int Np = P + 1;
+#pragma unroll
+  for (int c = 0; c < DIM + 2; ++c) {
+    double v[Np];
+#pragma unroll
+    for (int m = 0; m < Np; ++m) v[m] = rate[m][c];
+    line_move<Np>(L.x, from, fstride, to, tstride, v);
+#pragma unroll
+    for (int m = 0; m < Np; ++m) rate[m][c] = v[m];
+  }
 }
 
 // v of the lane N further in its row of 16 (cyclic)
@@ -345,72 +405,91 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) k_
   const int lane = threadIdx.x;
   const int el = min(lane / NL, EPW - 1);
   const int t = lane < EPW * NL ? lane % NL : 0;
-  const int eu = logical_block(a.xcd_remap) * EPW + el;
-  const int e = min(eu, a.ne - 1);
-  const bool valid = lane < EPW * NL && eu < a.ne;
+  const int e0 = logical_block(a.xcd_remap) * EPW;  // the wave's elements e0, ..., e0 + nv - 1
+  const int nv = min(EPW, a.ne - e0);
+  const int e = e0 + min(el, nv - 1);
+  const bool valid = lane < EPW * NL && el < nv;
   const long long Ntot = a.Ntot;
   const long long Gtot = (long long)a.ne * NFACE;
   const double *Vd = static_cast<const double *>(a.Vd);
   const double *Gf = static_cast<const double *>(a.Gf);
-  const unsigned xn = (unsigned)(e * ND + Np * t);  // first node of the lane's x-line
-  const int xs = el * NDS + (Np + 1) * t;           // the same, staged
-  const double Je = a.J[e];
-  int nbr[2 * DIM];
+  // nodes in memory order: lane + 64 m of the wave's contiguous EPW ND nodes
+  unsigned fn[Np];
+  int fx[Np];  // staged
 #pragma unroll
-  for (int f = 0; f < 2 * DIM; ++f) nbr[f] = a.nbr[e * 2 * DIM + f];
+  for (int m = 0; m < Np; ++m) {
+    const int k = lane + 64 * m, node = k % ND;
+    fn[m] = (unsigned)(e0 * ND + min(k, nv * ND - 1)) * 8u;
+    fx[m] = k / ND * NDS + node + node / Np;
+  }
+  const int le = min(el, nv - 1);  // e - e0
+  const auto mr = LineMeta<DIM, P>::load(a, e0, nv, lane);
 
-  // ---- the lane's x-line: state to LDS, indicator
-  double alpha = 0.0;
+  // ---- state to LDS, indicator
+  constexpr int NA = LineMeta<DIM, P>::Regs::NA;
   {
-    double f[Np], q[NQ][Np];
+    double nlr[NA];
+    double q[NQ][Np];
 #pragma unroll
     for (int c = 0; c < NQ; ++c)
 #pragma unroll
-      for (int m = 0; m < Np; ++m) q[c][m] = ld(a.U + c * Ntot, (xn + m) * 8u);
-    if (lane < EPW * NL) {
+      for (int m = 0; m < Np; ++m) q[c][m] = ld(a.U + c * Ntot, fn[m]);
+    L.m.store(mr, lane);
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
 #pragma unroll
-      for (int c = 0; c < NQ; ++c)
-#pragma unroll
-        for (int m = 0; m < Np; ++m) L.q[c][xs + m] = q[c][m];
+    for (int k = 0; k < NA; ++k) {
+      const int i = min(lane + 64 * k, nv * DIM * DIM - 1), r = i % (DIM * DIM);
+      nlr[k] = a.adj[(size_t)L.m.nbr[i / (DIM * DIM)][r / DIM * 2] * DIM * DIM + r];
     }
-    if (a.blending) {
-      // pressure * density = (gamma - 1) (rhoE rho - |m|^2/2)
 #pragma unroll
-      for (int m = 0; m < Np; ++m) {
-        double m2 = q[1][m] * q[1][m];
+    for (int c = 0; c < NQ; ++c)
 #pragma unroll
-        for (int d = 1; d < DIM; ++d) m2 = fma(q[1 + d][m], q[1 + d][m], m2);
-        f[m] = g.gammaM1 * fma(q[DIM + 1][m], q[0][m], -0.5 * m2);
-      }
-      alpha = line_alpha<DIM, P>(a, B, L.x, el, t, f);
-      if (valid && t == 0) a.alpha[e] = alpha;
+      for (int m = 0; m < Np; ++m)
+        if (64 * (m + 1) <= EPW * ND || lane + 64 * m < EPW * ND) L.q[c][fx[m]] = q[c][m];
+#pragma unroll
+    for (int k = 0; k < NA; ++k)
+      if (lane + 64 * k < EPW * DIM * DIM) (&L.nl[0][0])[lane + 64 * k] = nlr[k];
+  }
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  double alpha = 0.0;
+  if (a.blending) {
+    // pressure * density = (gamma - 1) (rhoE rho - |m|^2/2)
+    double f[Np];
+    const int xs = el * NDS + (Np + 1) * t;
+#pragma unroll
+    for (int m = 0; m < Np; ++m) {
+      double m2 = L.q[1][xs + m] * L.q[1][xs + m];
+#pragma unroll
+      for (int d = 1; d < DIM; ++d) m2 = fma(L.q[1 + d][xs + m], L.q[1 + d][xs + m], m2);
+      f[m] = g.gammaM1 * fma(L.q[DIM + 1][xs + m], L.q[0][xs + m], -0.5 * m2);
     }
+    alpha = line_alpha<DIM, P>(a, B, L.x, el, t, f);
+    if (valid && t == 0) a.alpha[e] = alpha;
   }
   __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
   const bool blend = a.blending && alpha > 1e-16;
   const double adg = blend ? 1.0 - alpha : 1.0;
 
-  // Running sums: the volume terms and, in the same units (-1/J times them is
-  // du/dt), the viscous divergence and the faces' lifted fluxes.
+  // running sums of the volume terms and the faces' lifted fluxes: -1/J times them is du/dt
   double rate[Np][NQ];
 #pragma unroll
   for (int m = 0; m < Np; ++m)
 #pragma unroll
-    for (int c = 0; c < NQ; ++c) rate[m][c] = VISC && c > 0 ? -Je * ld(Vd + (c - 1) * Ntot, (xn + m) * 8u) : 0.0;
+    for (int c = 0; c < NQ; ++c) rate[m][c] = 0.0;
   double D2[Np * Np];
 #pragma unroll
   for (int k = 0; k < Np * Np; ++k) D2[k] = B.Dhat2[k];
 
-  double xb[Np][NQ];
+  double xb[Np][NQ], vd[Np][VISC ? DIM + 1 : 1];
   // unrolled: in a rolled loop the constants of the branches rarely taken
   // (22 registers) stay live throughout
 #pragma unroll
   for (int d = 0; d < DIM; ++d) {
     const int lb = el * NDS + line_base<Np>(d, t), ls = line_stride<Np>(d);
-    const int nlo = nbr[2 * d], nhi = nbr[2 * d + 1];
+    const int nlo = L.m.nbr[le][2 * d], nhi = L.m.nbr[le][2 * d + 1];
     double met[DIM];
 #pragma unroll
-    for (int dd = 0; dd < DIM; ++dd) met[dd] = a.adj[(size_t)e * DIM * DIM + d * DIM + dd];
+    for (int dd = 0; dd < DIM; ++dd) met[dd] = L.m.adj[le][d * DIM + dd];
     // the two-point fluxes are linear in the metric: (1 - alpha) times the
     // volume terms of a blended element
     double metv[DIM];
@@ -422,9 +501,17 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) k_
     double gn[2][NVD];
 #pragma unroll
     for (int side = 0; side < 2; ++side) {
-      const unsigned nb = (unsigned)((side ? nhi : nlo) * ND + gb + (side ? 0 : (Np - 1) * gs[d]));
+      const int nbe = side ? nhi : nlo;
+      // a neighbour along x is mostly in the same wave
+      if (d == 0 && (unsigned)(nbe - e0) < (unsigned)nv) {
+        const int ns = (nbe - e0) * NDS + (Np + 1) * t + (side ? 0 : Np - 1);
 #pragma unroll
-      for (int c = 0; c < NQ; ++c) qn[side][c] = ld(a.U + c * Ntot, nb * 8u);
+        for (int c = 0; c < NQ; ++c) qn[side][c] = L.q[c][ns];
+      } else {
+        const unsigned nb = (unsigned)(nbe * ND + gb + (side ? 0 : (Np - 1) * gs[d]));
+#pragma unroll
+        for (int c = 0; c < NQ; ++c) qn[side][c] = ld(a.U + c * Ntot, nb * 8u);
+      }
       const unsigned fb = (unsigned)((side ? nhi : nlo) * NFACE + (2 * d + 1 - side) * NL + t);
 #pragma unroll
       for (int c = 0; c < NVD; ++c) gn[side][c] = VISC ? ld(Gf + c * Gtot, fb * 8u) : 0.0;
@@ -466,15 +553,19 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) k_
     double nl[DIM];
     if (d == DIM - 1) {
       // the RK base state (mode 2; in the other modes the stage state itself,
-      // a line already in cache)
+      // a line already in cache) and the viscous divergence
       const double *Xp = a.mode == 2 ? a.X : a.U;
 #pragma unroll
       for (int c = 0; c < NQ; ++c)
 #pragma unroll
-        for (int m = 0; m < Np; ++m) xb[m][c] = ld(Xp + c * Ntot, (xn + m) * 8u);
+        for (int m = 0; m < Np; ++m) xb[m][c] = ld(Xp + c * Ntot, fn[m]);
+#pragma unroll
+      for (int c = 0; c < (VISC ? NVD : 0); ++c)
+#pragma unroll
+        for (int m = 0; m < Np; ++m) vd[m][c] = ld(Vd + c * Ntot, fn[m]);
     }
 #pragma unroll
-    for (int dd = 0; dd < DIM; ++dd) nl[dd] = a.adj[(size_t)nlo * DIM * DIM + d * DIM + dd];
+    for (int dd = 0; dd < DIM; ++dd) nl[dd] = L.nl[le][d * DIM + dd];
 #pragma unroll
     for (int side = 0; side < 2; ++side) {
       const int m = side ? Np - 1 : 0;
@@ -501,18 +592,8 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) k_
         for (int c = 0; c < NQ; ++c) rate[m][c] += (side ? B.iw[0] : -B.iw[0]) * F[c];
       }
     }
-    // ---- the sums move to the next direction's lines (after the last, to the x-lines)
-    const int dn = d + 1 < DIM ? d + 1 : 0;
-    const int nb = el * NDS + line_base<Np>(dn, t), ns = line_stride<Np>(dn);
-#pragma unroll
-    for (int c = 0; c < NQ; ++c) {
-      double v[Np];
-#pragma unroll
-      for (int m = 0; m < Np; ++m) v[m] = rate[m][c];
-      line_move<Np>(L.x, lb, ls, nb, ns, v);
-#pragma unroll
-      for (int m = 0; m < Np; ++m) rate[m][c] = v[m];
-    }
+    // ---- the sums move to the next direction's lines
+    if (d + 1 < DIM) line_move_sums<DIM, P>(L, lb, ls, el * NDS + line_base<Np>(d + 1, t), line_stride<Np>(d + 1), rate);
   }
 
   // ---- subcell FV residual of the wave's blended elements (DGSEMIntegrator.hpp:
@@ -520,13 +601,13 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) k_
   //      fluxes (homogeneous in the normal) on top of the sums
   if (a.blending && __any(blend)) {
 #pragma unroll 1
-    for (int d = 0; d < DIM; ++d) {
+    for (int k = 0; k < DIM; ++k) {
+      const int d = k == 0 ? DIM - 1 : k - 1, dn = k;  // ends on the lines of the last direction, as it began
       const int lb = el * NDS + line_base<Np>(d, t), ls = line_stride<Np>(d);
-      const int dn = d + 1 < DIM ? d + 1 : 0;
       double n[DIM];
 #pragma unroll
       for (int dd = 0; dd < DIM; ++dd)
-        n[dd] = (blend ? alpha : 0.0) * a.adj[(size_t)e * DIM * DIM + d * DIM + dd];
+        n[dd] = (blend ? alpha : 0.0) * L.m.adj[le][d * DIM + dd];
       Pt<double, DIM> s[2];
       double F[2][NQ];
 #pragma unroll
@@ -553,29 +634,29 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) k_
           }
         }
       }
-      const int nb = el * NDS + line_base<Np>(dn, t), ns = line_stride<Np>(dn);
-#pragma unroll
-      for (int c = 0; c < NQ; ++c) {
-        double v[Np];
-#pragma unroll
-        for (int m = 0; m < Np; ++m) v[m] = rate[m][c];
-        line_move<Np>(L.x, lb, ls, nb, ns, v);
-#pragma unroll
-        for (int m = 0; m < Np; ++m) rate[m][c] = v[m];
-      }
+      line_move_sums<DIM, P>(L, lb, ls, el * NDS + line_base<Np>(dn, t), line_stride<Np>(dn), rate);
     }
   }
 
-  // ---- epilogue: dU, or the fused SSP-RK3 stage combination
-  if (!valid) return;
-  const double scale = -1.0 / Je;
+  // ---- epilogue, in memory order: dU, or the fused SSP-RK3 stage combination
+  const double scale = -1.0 / L.m.J[le];
+  const int lb = el * NDS + line_base<Np>(DIM - 1, t), ls = line_stride<Np>(DIM - 1);
 #pragma unroll
   for (int c = 0; c < NQ; ++c) {
+    if (lane < EPW * NL) {
+#pragma unroll
+      for (int m = 0; m < Np; ++m) L.x[lb + m * ls] = scale * rate[m][c];
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
 #pragma unroll
     for (int m = 0; m < Np; ++m) {
-      const unsigned byte = (xn + m) * 8u;
-      st(a.out + c * Ntot, byte, stage_value(a, dt, xb[m][c], L.q[c][xs + m], scale * rate[m][c]));
+      if (lane + 64 * m < nv * ND) {
+        double r = L.x[fx[m]];
+        if (VISC && c > 0) r += vd[m][VISC ? c - 1 : 0];
+        st(a.out + c * Ntot, fn[m], stage_value(a, dt, xb[m][c], L.q[c][fx[m]], r));
+      }
     }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
   }
 }
 
