@@ -500,6 +500,13 @@ static bool grad_line_form(const ShapeKernels *sk, const theseus_case_desc &d) {
   return true;
 }
 
+// The words a handle's or a pool's kernels share, in one allocation written at create
+struct SharedWords {
+  BasisArgs basis;
+  double pref;                         // mixed mode: background pressure, 0 before the first evaluation sets it
+  unsigned long long rates[kRateWords];  // stability rates
+};
+
 struct theseus_rhs {
   theseus_case_desc d;
   int Np, ndof, nfp, neq;
@@ -531,10 +538,11 @@ struct theseus_rhs {
   double *d_bc_data = nullptr;  // [max(num_bc, 1)][THESEUS_BC_DATA_STRIDE]
   double *d_alpha = nullptr;
   double *d_Fv = nullptr;       // NS: viscous volume divergence, then n.Fv at face points
-  double *d_pref = nullptr;     // mixed mode: background pressure (one double)
+  SharedWords *d_words = nullptr;
+  double *d_pref = nullptr;     // &d_words->pref
   bool pref_set = false;
   double *d_stage[2] = {nullptr, nullptr};
-  unsigned long long *d_rates = nullptr;
+  unsigned long long *d_rates = nullptr;  // d_words->rates
   double *d_meas = nullptr;           // integral measures: [nblocks][9] partials, then the 9 results
   double *d_ent = nullptr;            // entropy production: [nodes/256][2] partials, then the 2 results
   theseus_integral_measures diag0{};  // baseline: the first measures with nonzero mass
@@ -584,7 +592,7 @@ struct theseus_rhs {
     a.pref = d_pref;
     a.xcd_remap = nblocks() >= 256 ? kXcdRanges : 0;  // fewer blocks than CUs: the order only costs (8.5 us for 8.2 at 64 blocks)
     a.lte = ltev;
-    a.basis = basis;
+    a.basis = &d_words->basis;
     return a;
   }
   int nblocks() const { return (d.num_elements + sk->epb - 1) / sk->epb; }
@@ -988,14 +996,17 @@ static int create_impl(const theseus_case_desc *desc, const theseus_lte_table *l
 
   int rc = THESEUS_OK;
   const size_t M = (size_t)h->Ntot * h->neq;
-  if ((rc = upload(&h->d_J, d.elem_jac, ne)) || (rc = upload(&h->d_adj, d.elem_adj, (size_t)ne * dim * dim)) ||
+  SharedWords words{};
+  words.basis = h->basis;
+  if ((rc = upload(&h->d_words, &words, 1)) || (rc = upload(&h->d_J, d.elem_jac, ne)) || (rc = upload(&h->d_adj, d.elem_adj, (size_t)ne * dim * dim)) ||
       (rc = upload(&h->d_nbr, d.face_neighbor, (size_t)ne * 2 * dim)) ||
       (rc = upload_bc(&h->d_bc_type, &h->d_bc_data, d)) || (rc = upload<double>(&h->d_alpha, nullptr, ne)) ||
-      (rc = upload<unsigned long long>(&h->d_rates, nullptr, kRateWords)) || (rc = upload<double>(&h->d_pref, nullptr, 1)) ||
       (rc = upload<double>(&h->d_stage[0], nullptr, M)) || (rc = upload<double>(&h->d_stage[1], nullptr, M))) {
     theseus_rhs_destroy(h);
     return rc;
   }
+  h->d_pref = &h->d_words->pref;
+  h->d_rates = h->d_words->rates;
   if (d.flow_model == THESEUS_FLOW_NAVIER_STOKES) {
     const size_t nv = (size_t)(dim + 1) * ((size_t)h->Ntot + (size_t)ne * 2 * dim * h->nfp);
     if ((rc = upload<double>(&h->d_Fv, nullptr, nv))) {
@@ -1096,7 +1107,6 @@ static int create_impl(const theseus_case_desc *desc, const theseus_lte_table *l
   }
   h->d.elem_orient = nullptr;
   hipError_t e = hipMemset(h->d_alpha, 0, ne * sizeof(double));
-  if (e == hipSuccess) e = hipMemset(h->d_pref, 0, sizeof(double));  // defined before the first evaluation sets it
   if (e != hipSuccess) {
     theseus_rhs_destroy(h);
     return fail(THESEUS_ERR_DEVICE, std::string("hipMemset: ") + hipGetErrorString(e));
@@ -1159,7 +1169,6 @@ int theseus_rhs_destroy(theseus_rhs *h) {
   hipFree(h->d_bc_data);
   hipFree(h->d_alpha);
   hipFree(h->d_Fv);
-  hipFree(h->d_pref);
   hipFree(h->d_lte);
   hipFree(h->d_lte32);
   hipFree(h->d_lteT);
@@ -1171,7 +1180,7 @@ int theseus_rhs_destroy(theseus_rhs *h) {
   hipFree(h->d_ltebuckets);
   hipFree(h->d_stage[0]);
   hipFree(h->d_stage[1]);
-  hipFree(h->d_rates);
+  hipFree(h->d_words);
   hipFree(h->d_meas);
   hipFree(h->d_ent);
   hipFree(h->d_orient);
@@ -1721,7 +1730,8 @@ struct theseus_pool {
   int *d_bc_type = nullptr;
   double *d_bc_data = nullptr;
   double *d_case_dt = nullptr, *d_case_pref = nullptr;
-  unsigned long long *d_rates = nullptr;
+  SharedWords *d_words = nullptr;
+  unsigned long long *d_rates = nullptr;  // d_words->rates
   double *d_meas = nullptr;  // integral measures: partials of the largest case, then the results
   std::vector<PoolCase> cases;
   std::vector<unsigned char> slot_used;  // per element slot
@@ -1768,7 +1778,7 @@ struct theseus_pool {
     a.case_dt = d_case_dt;
     a.case_pref = d_case_pref;
     a.xcd_remap = xcd;
-    a.basis = basis;
+    a.basis = &d_words->basis;
     return a;
   }
 
@@ -2059,18 +2069,21 @@ int theseus_pool_create(const theseus_pool_desc *desc, theseus_pool **out) {
   int rc = THESEUS_OK;
   const size_t M = (size_t)p->Ntot * p->neq;
   const int dim = d.dim;
-  if ((rc = upload<double>(&p->d_J, nullptr, p->cap)) || (rc = upload<double>(&p->d_adj, nullptr, (size_t)p->cap * dim * dim)) ||
+  SharedWords words{};
+  words.basis = p->basis;
+  if ((rc = upload(&p->d_words, &words, 1)) || (rc = upload<double>(&p->d_J, nullptr, p->cap)) ||
+      (rc = upload<double>(&p->d_adj, nullptr, (size_t)p->cap * dim * dim)) ||
       (rc = upload<int>(&p->d_nbr, nullptr, (size_t)p->cap * 2 * dim)) ||
       (rc = upload<int>(&p->d_elem_case, nullptr, p->cap)) || (rc = upload<double>(&p->d_alpha, nullptr, p->cap)) ||
       (rc = upload<int>(&p->d_bc_type, nullptr, (size_t)d.max_cases * THESEUS_POOL_MAX_BC)) ||
       (rc = upload<double>(&p->d_bc_data, nullptr, (size_t)d.max_cases * THESEUS_POOL_MAX_BC * THESEUS_BC_DATA_STRIDE)) ||
       (rc = upload<double>(&p->d_case_dt, nullptr, d.max_cases)) ||
-      (rc = upload<double>(&p->d_case_pref, nullptr, d.max_cases)) ||
-      (rc = upload<unsigned long long>(&p->d_rates, nullptr, kRateWords)) || (rc = upload<double>(&p->d_U, nullptr, M)) ||
+      (rc = upload<double>(&p->d_case_pref, nullptr, d.max_cases)) || (rc = upload<double>(&p->d_U, nullptr, M)) ||
       (rc = upload<double>(&p->d_stage[0], nullptr, M)) || (rc = upload<double>(&p->d_stage[1], nullptr, M))) {
     theseus_pool_destroy(p);
     return rc;
   }
+  p->d_rates = p->d_words->rates;
   if (d.flow_model == THESEUS_FLOW_NAVIER_STOKES &&
       (rc = upload<double>(&p->d_Fv, nullptr, (size_t)(dim + 1) * ((size_t)p->Ntot + (size_t)p->cap * 2 * dim * p->nfp)))) {
     theseus_pool_destroy(p);
@@ -2137,7 +2150,7 @@ int theseus_pool_destroy(theseus_pool *p) {
   hipFree(p->d_alpha);
   hipFree(p->d_case_dt);
   hipFree(p->d_case_pref);
-  hipFree(p->d_rates);
+  hipFree(p->d_words);
   hipFree(p->d_meas);
   hipFree(p->d_U);
   hipFree(p->d_stage[0]);

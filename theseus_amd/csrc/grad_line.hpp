@@ -40,7 +40,7 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) k_
   __shared__ GradLineLds<DIM, P> L;
 
   const GasC<double> &g = a.gas;
-  const BasisArgs &B = a.basis;
+  ConstBasis &B = const_basis(a.basis);
   const int lane = threadIdx.x;
   const int el = min(lane / NL, EPW - 1);
   const int t = lane < EPW * NL ? lane % NL : 0;

@@ -305,7 +305,7 @@ __device__ __forceinline__ double row_rotate(double v) {
 // x-line nodes.  The sums over an element's modes pair the operands as
 // blending_alpha's tree does where its lines fill a power of two of lanes.
 template <int DIM, int P>
-__device__ __forceinline__ double line_alpha(const RHSCore &a, const BasisArgs &B, double *buf, int el, int t, double *f) {
+__device__ __forceinline__ double line_alpha(const RHSCore &a, ConstBasis &B, double *buf, int el, int t, double *f) {
   using S = LineShape<DIM, P>;
   constexpr int Np = S::Np, NL = S::NL, NDS = S::NDS;
   auto sweep = [&] {
@@ -401,7 +401,7 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) k_
   const double dt = a.case_dt ? a.case_dt[0] : a.dt;
   if (a.mode != 0 && a.case_dt && dt == 0.0) return;
   const GasC<double> &g = a.gas;
-  const BasisArgs &B = a.basis;
+  ConstBasis &B = const_basis(a.basis);
   const int lane = threadIdx.x;
   const int el = min(lane / NL, EPW - 1);
   const int t = lane < EPW * NL ? lane % NL : 0;

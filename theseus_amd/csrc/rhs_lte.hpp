@@ -95,7 +95,7 @@ __global__ void __launch_bounds__((Shape<DIM, P>::TPB)) k_rhs_lte(RHSArgs a) {
 #pragma unroll
   for (int q = 0; q < NQ; ++q) qown[q] = a.U[q * Ntot + ebase];
   static_assert(Np * Np <= TPB, "one basis entry per lane");
-  const double bD2 = a.basis.Dhat2[min(tid, Np * Np - 1)];
+  const double bD2 = const_basis(a.basis).Dhat2[min(tid, Np * Np - 1)];
   meta_load_normals<DIM, EPB, TPB>(a, ebase_blk, mr);
   if (tid < Np * Np) sD2[tid] = R(bD2);
 
@@ -226,7 +226,7 @@ __global__ void __launch_bounds__((Shape<DIM, P>::TPB)) k_rhs_lte(RHSArgs a) {
 
   // ---- faces (EulerOperator_impl.hpp:211-392)
   {
-    const double w0 = a.basis.w[0];
+    const double w0 = const_basis(a.basis).w[0];
 #pragma unroll
     for (int r = 0; r < NFR; ++r) {
       const int fi = tid + r * TPB;
@@ -406,7 +406,7 @@ __attribute__((amdgpu_waves_per_eu(LteecWaves<R, DIM, P, VISC>::value))) k_rhs_l
 #pragma unroll
   for (int q = 0; q < NQ; ++q) qown[q] = a.U[q * Ntot + ebase];
   static_assert(Np * Np <= TPB, "one basis entry per lane");
-  const double bD2 = a.basis.Dhat2[min(tid, Np * Np - 1)];
+  const double bD2 = const_basis(a.basis).Dhat2[min(tid, Np * Np - 1)];
   meta_load_normals<DIM, EPB, TPB>(a, ebase_blk, mr);
   if (tid < Np * Np) sD2[tid] = R(bD2);
   meta_store<DIM, EPB, TPB>(mr, sm);
@@ -525,7 +525,7 @@ __attribute__((amdgpu_waves_per_eu(LteecWaves<R, DIM, P, VISC>::value))) k_rhs_l
   for (int q = 0; q < NQ; ++q) du[q] = R(-1.0 / Je) * rate[q];
 
   // ---- faces (EulerOperator_impl.hpp:211-392)
-  const double w0 = a.basis.w[0];
+  const double w0 = const_basis(a.basis).w[0];
 #pragma unroll 1
   for (int r = 0; r < NFR; ++r) {
     const int fi = tid + r * TPB;
