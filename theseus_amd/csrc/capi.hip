@@ -593,6 +593,7 @@ struct theseus_rhs {
     a.xcd_remap = nblocks() >= 256 ? kXcdRanges : 0;  // fewer blocks than CUs: the order only costs (8.5 us for 8.2 at 64 blocks)
     a.lte = ltev;
     a.basis = &d_words->basis;
+    std::memcpy(a.w, basis.w, sizeof a.w);
     return a;
   }
   int nblocks() const { return (d.num_elements + sk->epb - 1) / sk->epb; }
@@ -1779,6 +1780,7 @@ struct theseus_pool {
     a.case_pref = d_case_pref;
     a.xcd_remap = xcd;
     a.basis = &d_words->basis;
+    std::memcpy(a.w, basis.w, sizeof a.w);
     return a;
   }
 
