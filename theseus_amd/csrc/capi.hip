@@ -348,36 +348,50 @@ __global__ void __launch_bounds__(256) k_sum_pairs_final(const double *partial, 
   if (tid < 2) out[tid] = red[0][tid];
 }
 
-// rates[q] = max over the slots of rate q (one 64-lane workgroup).
-__global__ void __launch_bounds__(64) k_rates_fold(unsigned long long *rates) {
-  const int t = threadIdx.x;
+// The rates of a stability estimate -- the maxima over the slots, the same in
+// all lanes of the one wave that calls this -- leaving the slots zero for the
+// next one.  What consumes an estimate takes them itself, so an estimate costs
+// no launches to clear and to fold the slots (3.5 us of a variable step on
+// 256 elements).
+__device__ __forceinline__ void take_rates(unsigned long long *rates, double (&r)[3]) {
+  static_assert(kRateSlots == 64, "a slot a lane");
 #pragma unroll
   for (int q = 0; q < 3; ++q) {
-    unsigned long long v = t < kRateSlots ? rates[3 + q * kRateSlots + t] : 0ull;
+    unsigned long long *slot = rates + 3 + q * kRateSlots + threadIdx.x;
+    unsigned long long v = *slot;
+    *slot = 0ull;
     // non-negative doubles order like their bit patterns
     for (int off = 32; off > 0; off >>= 1) {
       const unsigned long long o = __shfl_xor(v, off, 64);
       v = o > v ? o : v;
     }
-    if (t == 0) rates[q] = v;
+    r[q] = __longlong_as_double((long long)v);
   }
 }
 
-__global__ void k_zero_u64(unsigned long long *p, int n) {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t < n) p[t] = 0ull;
+// rates[0..2], for the host
+__global__ void __launch_bounds__(64) k_rates(unsigned long long *rates) {
+  double r[3];
+  take_rates(rates, r);
+#pragma unroll
+  for (int q = 0; q < 3; ++q)
+    if (threadIdx.x == 0) rates[q] = (unsigned long long)__double_as_longlong(r[q]);
 }
 
 // Background pressure of the mixed mode: the pressure of the first node of
 // the state (one lane; a vector store).
 template <int DIM>
-__global__ void k_pref(const double *U, long long Ntot, GasC<double> g, double *out) {
-  if (blockIdx.x != 0 || threadIdx.x != 0) return;
+__device__ __forceinline__ double first_pressure(const double *U, long long Ntot, const GasC<double> &g) {
   Pt<double, DIM> s;
 #pragma unroll
   for (int q = 0; q < DIM + 2; ++q) s.q[q] = U[q * Ntot];
   derive(g, s);
-  out[0] = s.p;
+  return s.p;
+}
+template <int DIM>
+__global__ void k_pref(const double *U, long long Ntot, GasC<double> g, double *out) {
+  if (blockIdx.x != 0 || threadIdx.x != 0) return;
+  out[0] = first_pressure<DIM>(U, Ntot, g);
 }
 
 // ---------------------------------------------------------------------------
@@ -504,7 +518,7 @@ static bool grad_line_form(const ShapeKernels *sk, const theseus_case_desc &d) {
 struct SharedWords {
   BasisArgs basis;
   double pref;                         // mixed mode: background pressure, 0 before the first evaluation sets it
-  unsigned long long rates[kRateWords];  // stability rates
+  unsigned long long rates[kRateWords];  // stability rates, zero before an estimate
 };
 
 struct theseus_rhs {
@@ -889,6 +903,56 @@ static int lte_lookups(theseus_rhs *h, const theseus_lte_table *lt) {
   return THESEUS_OK;
 }
 
+// A pooled case's time step from its stability rates, cfl / total rate, or 0
+// (the case does not advance) when the rate is not positive and finite; and,
+// in the mixed mode, its background pressure, that of its first node (U).
+template <int DIM>
+__global__ void __launch_bounds__(64) k_case_start(unsigned long long *rates, double cfl, double *dt, const double *U,
+                                                   long long Ntot, GasC<double> g, double *pref) {
+  double r[3];
+  take_rates(rates, r);
+  if (threadIdx.x != 0) return;
+  const double rate = fmax(r[0], r[1]) + r[2];
+  dt[0] = (rate > 0.0 && isfinite(rate)) ? cfl / rate : 0.0;
+  pref[0] = first_pressure<DIM>(U, Ntot, g);
+}
+
+// dst[q dstride + i] = src[q sstride + i], i < n, q = blockIdx.y: the fields of
+// a case between a vector and the pool in one launch (a copy per field: five
+// commands of 4 us)
+__global__ void __launch_bounds__(256) k_copy_fields(double *dst, long long dstride, const double *src,
+                                                     long long sstride, long long n) {
+  const long long i = (long long)blockIdx.x * 256 + threadIdx.x;
+  if (i < n) dst[blockIdx.y * dstride + i] = src[blockIdx.y * sstride + i];
+}
+
+// A case's geometry and connectivity from the pinned staging buffer to its slots
+__global__ void __launch_bounds__(256) k_case_mesh(double *J, double *adj, int *nbr, const double *hJ,
+                                                   const double *hA, const int *hN, int nJ, int nA, int nN) {
+  const int i = blockIdx.x * 256 + threadIdx.x;
+  if (i < nJ) J[i] = hJ[i];
+  if (i < nA) adj[i] = hA[i];
+  if (i < nN) nbr[i] = hN[i];
+}
+
+// The fields of a case, in one launch where the caller's end (user) is memory of the device too
+static int copy_fields(double *dst, long long dstride, const double *src, long long sstride, long long n, int neq,
+                       const double *user, hipStream_t s) {
+  int device = 0;
+  HIP_TRY(hipGetDevice(&device));
+  hipPointerAttribute_t at;
+  if (hipPointerGetAttributes(&at, user) == hipSuccess && at.type == hipMemoryTypeDevice && at.device == device) {
+    hipLaunchKernelGGL(k_copy_fields, dim3((unsigned)((n + 255) / 256), neq), dim3(256), 0, s, dst, dstride, src,
+                       sstride, n);
+    HIP_TRY(hipGetLastError());
+    return THESEUS_OK;
+  }
+  (void)hipGetLastError();  // an unregistered host pointer
+  for (int q = 0; q < neq; ++q)
+    HIP_TRY(hipMemcpyAsync(dst + q * dstride, src + q * sstride, n * sizeof(double), hipMemcpyDefault, s));
+  return THESEUS_OK;
+}
+
 extern "C" {
 
 const char *theseus_last_error(void) { return g_last_error.c_str(); }
@@ -1243,9 +1307,8 @@ static int enqueue_ssprk3(theseus_rhs *h, double *u, double dt, const double *dt
   return enqueue_rhs(h, a, s);
 }
 
-// Zeroes the rate slots and launches the stability kernel (no host copy).
+// Launches the stability kernel; a kernel that takes its rates (take_rates) follows it.
 static void enqueue_stability(theseus_rhs *h, const double *u, hipStream_t s) {
-  hipLaunchKernelGGL(k_zero_u64, dim3((kRateWords + 63) / 64), dim3(64), 0, s, h->d_rates, kRateWords);
   StabArgs a;
   std::memset(&a, 0, sizeof(a));
   a.U = u;
@@ -1274,17 +1337,15 @@ static void enqueue_stability(theseus_rhs *h, const double *u, hipStream_t s) {
     a.lte_nodes = 1;
   }
   h->sk->stability(a, h->nblocks(), s);
-  hipLaunchKernelGGL(k_rates_fold, dim3(1), dim3(64), 0, s, h->d_rates);
 }
 
 // The variable-step decision of src/Simulation.cpp:1136-1158,1240-1301 and
 // TimeStepControl.hpp:15-48 on the device, from the rates just estimated.
-__global__ void k_clock(theseus_clock *c, const unsigned long long *rates) {
+__global__ void __launch_bounds__(64) k_clock(theseus_clock *c, unsigned long long *rates) {
+  double r[3];
+  take_rates(rates, r);
   if (threadIdx.x != 0) return;
-  const double adv = __longlong_as_double((long long)rates[0]);
-  const double surf = __longlong_as_double((long long)rates[1]);
-  const double diff = __longlong_as_double((long long)rates[2]);
-  const double rate = fmax(adv, surf) + diff;  // StabilityEstimate::TotalRate
+  const double rate = fmax(r[0], r[1]) + r[2];  // StabilityEstimate::TotalRate
   c->rate = rate;
   if (!(rate > 0.0) || !isfinite(rate)) {
     c->dt_real = 0.0;
@@ -1304,17 +1365,6 @@ __global__ void k_clock(theseus_clock *c, const unsigned long long *rates) {
   c->dt_real = dt_real;
   c->t = t + dt_real;
   if (dt_real > 0.0) c->steps += 1;
-}
-
-// A pooled case's time step from its stability rates: cfl / total rate, or 0
-// (the case does not advance) when the rate is not positive and finite.
-__global__ void k_case_dt(const unsigned long long *rates, double cfl, double *dt) {
-  if (threadIdx.x != 0) return;
-  const double adv = __longlong_as_double((long long)rates[0]);
-  const double surf = __longlong_as_double((long long)rates[1]);
-  const double diff = __longlong_as_double((long long)rates[2]);
-  const double rate = fmax(adv, surf) + diff;
-  dt[0] = (rate > 0.0 && isfinite(rate)) ? cfl / rate : 0.0;
 }
 
 int theseus_rhs_step_ssprk3(theseus_rhs *h, double *u, double t, double dt, void *stream) {
@@ -1472,6 +1522,7 @@ int theseus_rhs_estimate_stability(theseus_rhs *h, const double *u, theseus_stab
   const int rc = aligned_input(h, u, &ua, s);
   if (rc) return rc;
   enqueue_stability(h, ua, s);
+  hipLaunchKernelGGL(k_rates, dim3(1), dim3(64), 0, s, h->d_rates);
   HIP_TRY(hipGetLastError());
   unsigned long long r[3];
   HIP_TRY(hipMemcpyAsync(r, h->d_rates, sizeof r, hipMemcpyDeviceToHost, s));
@@ -2239,15 +2290,14 @@ int theseus_pool_admit(theseus_pool *p, const theseus_case_desc *c, const double
     HIP_TRY(hipMemcpyAsync(p->d_bc_data + (size_t)boff * THESEUS_BC_DATA_STRIDE, hB, nB * sizeof(double),
                            hipMemcpyHostToDevice, s));
   }
-  HIP_TRY(hipMemcpyAsync(p->d_J + start, hJ, nJ * sizeof(double), hipMemcpyHostToDevice, s));
-  HIP_TRY(hipMemcpyAsync(p->d_adj + (size_t)start * dim * dim, hA, nA * sizeof(double), hipMemcpyHostToDevice, s));
-  HIP_TRY(hipMemcpyAsync(p->d_nbr + (size_t)start * 2 * dim, hN, nN * sizeof(int), hipMemcpyHostToDevice, s));
+  hipLaunchKernelGGL(k_case_mesh, dim3((unsigned)((std::max(nA, nN) + 255) / 256)), dim3(256), 0, s, p->d_J + start,
+                     p->d_adj + (size_t)start * dim * dim, p->d_nbr + (size_t)start * 2 * dim, hJ, hA, hN, (int)nJ,
+                     (int)nA, (int)nN);
+  HIP_TRY(hipGetLastError());
   HIP_TRY(hipEventRecord(staged, s));
   const long long nd = (long long)ne * p->ndof, off = (long long)start * p->ndof;
-  for (int q = 0; q < p->neq; ++q)
-    HIP_TRY(hipMemcpyAsync(p->d_U + q * p->Ntot + off, u0 + q * nd, nd * sizeof(double), hipMemcpyDefault, s));
+  if ((rc = copy_fields(p->d_U + off, p->Ntot, u0, nd, nd, p->neq, u0, s))) return rc;
   // stability estimate of the case alone (its element range), then dt and the background pressure
-  hipLaunchKernelGGL(k_zero_u64, dim3((kRateWords + 63) / 64), dim3(64), 0, s, p->d_rates, kRateWords);
   StabArgs a;
   std::memset(&a, 0, sizeof(a));
   a.U = p->d_U;
@@ -2267,10 +2317,8 @@ int theseus_pool_admit(theseus_pool *p, const theseus_case_desc *c, const double
   a.gas = p->gas;
   a.w0 = p->basis.w[0];
   p->sk->stability(a, (ne + p->sk->epb - 1) / p->sk->epb, s);
-  hipLaunchKernelGGL(k_rates_fold, dim3(1), dim3(64), 0, s, p->d_rates);
-  if (dim == 2) hipLaunchKernelGGL(k_pref<2>, dim3(1), dim3(64), 0, s, p->d_U + off, p->Ntot, p->gas, p->d_case_pref + cid);
-  else hipLaunchKernelGGL(k_pref<3>, dim3(1), dim3(64), 0, s, p->d_U + off, p->Ntot, p->gas, p->d_case_pref + cid);
-  hipLaunchKernelGGL(k_case_dt, dim3(1), dim3(64), 0, s, p->d_rates, cfl, p->d_case_dt + cid);
+  hipLaunchKernelGGL(dim == 2 ? k_case_start<2> : k_case_start<3>, dim3(1), dim3(64), 0, s, p->d_rates, cfl,
+                     p->d_case_dt + cid, p->d_U + off, p->Ntot, p->gas, p->d_case_pref + cid);
   hipLaunchKernelGGL(k_fill_i32, dim3((ne + 255) / 256), dim3(256), 0, s, p->d_elem_case + start, ne, cid);
   HIP_TRY(hipGetLastError());
   double dt = 0.0;
@@ -2439,8 +2487,8 @@ int theseus_pool_read(theseus_pool *p, int case_id, double *u, void *stream) {
   const PoolCase &c = p->cases[case_id];
   const long long nd = (long long)c.ne * p->ndof, off = (long long)c.start * p->ndof;
   hipStream_t s = (hipStream_t)stream;
-  for (int q = 0; q < p->neq; ++q)
-    HIP_TRY(hipMemcpyAsync(u + q * nd, p->d_U + q * p->Ntot + off, nd * sizeof(double), hipMemcpyDefault, s));
+  const int rc = copy_fields(u, nd, p->d_U + off, p->Ntot, nd, p->neq, u, s);
+  if (rc) return rc;
   HIP_TRY(hipStreamSynchronize(s));
   return THESEUS_OK;
 }

@@ -1548,7 +1548,7 @@ __attribute__((amdgpu_waves_per_eu(GradWaves<R, DIM, P, EPBX, BND, LTE>::value))
 // ---------------------------------------------------------------------------
 // Stability rates buffer: [0..2] the advective, surface and diffusive rate
 // (bit patterns of non-negative doubles), then kRateSlots partial maxima of
-// each, zeroed before and folded after each estimate.
+// each, zero before an estimate; what takes its rates leaves them zero.
 constexpr int kRateSlots = 64;
 constexpr int kRateWords = 3 + 3 * kRateSlots;
 
@@ -1710,7 +1710,7 @@ __global__ void __launch_bounds__((Shape<DIM, P>::TPB)) k_stability(StabArgs a) 
   diff = wave_max(diff);
   if ((threadIdx.x & 63) == 0) {
     // one of kRateSlots slots per rate (by block), so that the grid's
-    // atomics do not all queue on three addresses; k_rates_fold takes the max
+    // atomics do not all queue on three addresses; take_rates takes the max
     unsigned long long *slot = a.rates + 3 + (blockIdx.x % kRateSlots);
     atomicMax(slot, (unsigned long long)__double_as_longlong(adv));
     atomicMax(slot + kRateSlots, (unsigned long long)__double_as_longlong(surf));
