@@ -1,14 +1,15 @@
-"""The line forms of the fused kernel and the gradient pass (FP64, meshes
-without boundary faces, enough elements to fill the chip) against the CPU
-oracle, at the element counts from which they are used (odd counts: the last wave is partly filled), on states that
-take each branch of the logarithmic means, with and without blended elements.
-The bound is that of the other FP64 RHS tests, relative L2 <= 1e-12."""
+"""The line forms of the fused kernel and the gradient pass (FP64, enough
+elements to fill the chip) against the CPU oracle, at the element counts from
+which they are used (odd counts: the last wave is partly filled), on states
+that take each branch of the logarithmic means, with and without blended
+elements.  The bound is that of the other FP64 RHS tests, relative L2 <= 1e-12."""
 import numpy as np
 import pytest
 
 from theseus_amd import _abi as A
 
 from .gpu_helpers import gpu_rhs, make_case, oracle_case, rel_l2, smooth_state
+from .test_gpu_bc import _case as _bc_case
 
 pytestmark = pytest.mark.gpu
 
@@ -42,6 +43,23 @@ def _state(mesh, order, gamma, noise):
 def test_line_form_fp64(oracle, dim, n, order, pairing, visc, blending, noise):
     flow = A.FLOW_NAVIER_STOKES if visc else A.FLOW_EULER
     rt, mesh = make_case(dim, order, n, pairing, flow=flow, blending=blending)
+    U = _state(mesh, order, rt.gamma, noise)
+    ref = oracle_case(oracle, rt, mesh).rhs(U)
+    got, _ = gpu_rhs(rt, mesh, U)
+    assert rel_l2(got, ref) <= 1e-12, rel_l2(got, ref)
+
+
+@pytest.mark.parametrize("noise", ["short", "far"])
+@pytest.mark.parametrize("blending", [False, True])
+@pytest.mark.parametrize("kind", ["euler", "no_slip"])
+@pytest.mark.parametrize("dim,n,order,pairing,periodic", [
+    (2, (147, 147), 2, "roe", False), (2, (129, 128), 3, "ranocha_llf", (True, False)), (2, (111, 111), 4, "hll", False),
+    (3, (20, 19, 19), 2, "chandrashekar", False), (3, (13, 13, 13), 3, "ranocha_llf", (False, True, False)),
+    (3, (17, 16, 16), 4, "llf", False),
+])
+def test_line_form_boundaries(oracle, dim, n, order, pairing, periodic, kind, blending, noise):
+    """Every boundary type of the Euler equations on the sides of a box"""
+    rt, mesh = _bc_case(dim, order, n, pairing, A.FLOW_EULER, kind, blending=blending, periodic=periodic)
     U = _state(mesh, order, rt.gamma, noise)
     ref = oracle_case(oracle, rt, mesh).rhs(U)
     got, _ = gpu_rhs(rt, mesh, U)

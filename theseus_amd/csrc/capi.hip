@@ -489,8 +489,8 @@ static bool line_offsets(int ne, int ndof, int dim, int nfp) {
 
 // Does the fused kernel run in its line form on ne elements?  Where it is
 // built, on enough waves to fill the chip (line_min_waves).
-static bool line_form(const FluxKernels *fk, bool ns, int ne) {
-  if (!fk || !(ns ? fk->ns_line : fk->euler_line)) return false;
+static bool line_form(const FluxKernels *fk, bool ns, bool boundary, int ne) {
+  if (!fk || !(ns ? (boundary ? nullptr : fk->ns_line) : fk->euler_line[boundary])) return false;
   return (ne + fk->line_epw - 1) / fk->line_epw >= (ns ? fk->ns_line_min : fk->euler_line_min);
 }
 
@@ -504,6 +504,7 @@ static bool grad_line_form(const ShapeKernels *sk, const theseus_case_desc &d) {
     for (int k = 0; k < dim; ++k) {
       const double *own = d.elem_adj + (e * dim + k) * dim;
       const double *low = d.elem_adj + ((long long)d.face_neighbor[e * 2 * dim + 2 * k] * dim + k) * dim;
+      if (std::equal(own, own + dim, low)) continue;
       double diff = 0.0, size = 0.0;
       for (int c = 0; c < dim; ++c) {
         diff += std::fabs(own[c] - low[c]);
@@ -664,7 +665,7 @@ static int enqueue_rhs(theseus_rhs *h, RHSArgs a, hipStream_t s) {
     if (ns) a.xcd_remap ^= kReverse;
     if (h->line) {
       const int nl = (h->d.num_elements + h->fk->line_epw - 1) / h->fk->line_epw;
-      timed(h, 0, s, [&] { (ns ? h->fk->ns_line : h->fk->euler_line)(a, nl, s); });
+      timed(h, 0, s, [&] { (ns ? h->fk->ns_line : h->fk->euler_line[h->has_boundary])(a, nl, s); });
     } else {
       timed(h, 0, s, [&] { (ns ? h->fk->ns : h->fk->euler)[h->pm][h->has_boundary](a, nb, s); });
     }
@@ -1050,10 +1051,10 @@ static int create_impl(const theseus_case_desc *desc, const theseus_lte_table *l
   legendre_vandermonde_inverse(d.order, x, h->basis.Vinv);
   init_gas(d, h->gas, h->gas32);
   h->pm = d.precision == THESEUS_PRECISION_MIXED ? 1 : 0;
-  if (!has_boundary && !lk && h->pm == 0 && line_offsets(ne, h->ndof, dim, h->nfp)) {
+  if (!lk && h->pm == 0 && line_offsets(ne, h->ndof, dim, h->nfp)) {
     const bool ns = d.flow_model == THESEUS_FLOW_NAVIER_STOKES;
-    h->line = line_form(fk, ns, ne);
-    h->grad_line = ns && grad_line_form(sk, d);
+    h->line = line_form(fk, ns, has_boundary, ne);
+    h->grad_line = ns && !has_boundary && grad_line_form(sk, d);
   }
   h->adv_scale = advection_scale(d.order);
   h->diff_scale = diffusion_scale(d.order);

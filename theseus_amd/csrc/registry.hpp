@@ -23,9 +23,9 @@ using MeasLaunch = void (*)(const MeasArgs &, int nblocks, hipStream_t);
 struct FluxKernels {
   RHSLaunch euler[2][2] = {};  // fused volume + face
   RHSLaunch ns[2][2] = {};     // Navier-Stokes pass 2
-  // the FP64 line form (k_rhs_line) on meshes without boundary faces, and the
+  // the FP64 line form (k_rhs_line) on meshes without ([0]) and with boundary faces (Euler), and the
   // fewest workgroups (waves of line_epw elements) it is used from; null where it is not built
-  RHSLaunch euler_line = nullptr, ns_line = nullptr;
+  RHSLaunch euler_line[2] = {}, ns_line = nullptr;
   int euler_line_min = 0, ns_line_min = 0;
   int line_epw = 0;
 };
@@ -129,20 +129,25 @@ void launch_measures(const MeasArgs &a, int nb, hipStream_t s) {
 // sets of sums, the ratios at p = 3 were 1.03 1.06 1.33 1.14 for Euler and 0.96
 // 0.98 1.14 1.02 for NS, at p = 4 0.81 0.89 1.15 1.09 and 0.82 0.96 1.10 1.04,
 // and a pool's results would depend on its launch range: FP64 only.
+// With boundary faces (Euler; at 1024, 2048 and 4096 waves): 2-D Ranocha/LLF
+// p = 3 1.07 1.27 1.18, p = 4 1.14 1.25 1.47, central/HLL p = 4 1.26 1.25 1.42;
+// 3-D Ranocha/LLF p = 3 1.43 1.74 1.68, central/HLL p = 2 1.01 1.41 1.26; but
+// Chandrashekar's 2-D p = 3 1.01 1.06 0.99 and p = 4 0.98 0.96 1.13, left out,
+// as are central/LLF and central/Roe in 3-D at p = 4 (332 and 424 B of scratch).
 template <int DIM, int P, int VOL, int SURF>
-constexpr int line_min_waves(bool visc) {
+constexpr int line_min_waves(bool visc, bool boundary = false) {
   if (P < 2 || P > 4 || VOL == 3) return 0;
   if (DIM == 3 && P == 4) {
-    if (VOL == 1 || (VOL == 0 && SURF != 5 && visc)) return 0;
+    if (VOL == 1 || (VOL == 0 && (visc ? SURF != 5 : boundary && SURF != 4))) return 0;
     return VOL == 2 && (!visc || SURF == 5) ? 1024 : 2048;
   }
-  if (DIM == 2 && P == 4 && VOL == 1 && visc) return 0;
+  if (DIM == 2 && VOL == 1 && ((P == 4 && visc) || (P >= 3 && boundary))) return 0;
   return DIM == 3 && (SURF == 5 || (P == 3 && !visc)) ? 512 : 1024;
 }
 
-template <int DIM, int P, int VOL, int SURF, bool VISC>
+template <int DIM, int P, int VOL, int SURF, bool VISC, bool BND = false>
 void launch_rhs_line(const RHSArgs &a, int nb, hipStream_t s) {
-  hipLaunchKernelGGL((k_rhs_line<DIM, P, VOL, SURF, VISC>), dim3(nb), dim3(64), 0, s, a);
+  hipLaunchKernelGGL((k_rhs_line<DIM, P, VOL, SURF, VISC, BND>), dim3(nb), dim3(64), 0, s, a);
 }
 
 template <int DIM, int VOL, int SURF, int P>
@@ -150,7 +155,9 @@ struct FluxRegistrar {
   FluxRegistrar() {
     FluxKernels k;
     if constexpr (line_min_waves<DIM, P, VOL, SURF>(false) > 0) {
-      k.euler_line = &launch_rhs_line<DIM, P, VOL, SURF, false>;
+      k.euler_line[0] = &launch_rhs_line<DIM, P, VOL, SURF, false>;
+      if constexpr (line_min_waves<DIM, P, VOL, SURF>(false, true) > 0)
+        k.euler_line[1] = &launch_rhs_line<DIM, P, VOL, SURF, false, true>;
       k.euler_line_min = line_min_waves<DIM, P, VOL, SURF>(false);
       k.line_epw = LineShape<DIM, P>::EPW;
     }

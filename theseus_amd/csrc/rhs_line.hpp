@@ -387,10 +387,11 @@ __device__ __forceinline__ void st(T *base, unsigned byte, T v) {
   *reinterpret_cast<T *>(reinterpret_cast<char *>(base) + byte) = v;
 }
 
-// Meshes without boundary faces whose fields and n.Fv rows can be addressed
-// with 32-bit byte offsets.
-template <int DIM, int P, int VOL, int SURF, bool VISC>
+// Meshes whose fields and n.Fv rows can be addressed with 32-bit byte offsets;
+// BND: with boundary faces (Euler).
+template <int DIM, int P, int VOL, int SURF, bool VISC, bool BND = false>
 __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) k_rhs_line(RHSArgs a) {
+  static_assert(!(VISC && BND), "boundary faces: Euler");
   using S = LineShape<DIM, P>;
   constexpr int Np = S::Np, NL = S::NL, ND = S::ND, NQ = S::NQ, EPW = S::EPW, NDS = S::NDS;
   constexpr int NVD = DIM + 1;
@@ -439,7 +440,8 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) k_
 #pragma unroll
     for (int k = 0; k < NA; ++k) {
       const int i = min(lane + 64 * k, nv * DIM * DIM - 1), r = i % (DIM * DIM);
-      nlr[k] = a.adj[(size_t)L.m.nbr[i / (DIM * DIM)][r / DIM * 2] * DIM * DIM + r];
+      const int nb = L.m.nbr[i / (DIM * DIM)][r / DIM * 2];
+      nlr[k] = a.adj[(size_t)(BND && nb < 0 ? e0 + i / (DIM * DIM) : nb) * DIM * DIM + r];
     }
 #pragma unroll
     for (int c = 0; c < NQ; ++c)
@@ -502,8 +504,12 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) k_
 #pragma unroll
     for (int side = 0; side < 2; ++side) {
       const int nbe = side ? nhi : nlo;
-      // a neighbour along x is mostly in the same wave
-      if (d == 0 && (unsigned)(nbe - e0) < (unsigned)nv) {
+      // a neighbour along x is mostly in the same wave; a boundary point
+      // takes the element's own trace
+      if (BND && nbe < 0) {
+#pragma unroll
+        for (int c = 0; c < NQ; ++c) qn[side][c] = L.q[c][lb + (side ? Np - 1 : 0) * ls];
+      } else if (d == 0 && (unsigned)(nbe - e0) < (unsigned)nv) {
         const int ns = (nbe - e0) * NDS + (Np + 1) * t + (side ? 0 : Np - 1);
 #pragma unroll
         for (int c = 0; c < NQ; ++c) qn[side][c] = L.q[c][ns];
@@ -569,7 +575,26 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) k_
 #pragma unroll
     for (int side = 0; side < 2; ++side) {
       const int m = side ? Np - 1 : 0;
-      const double *n = side ? met : nl;
+      // a boundary point evaluates F*(q, q_ext, n_out) with the interior trace
+      // first, or the wall flux (0, p* n_out, 0) (bc_kernels.hpp:138-287)
+      const int nbe = side ? nhi : nlo;
+      const bool bdr = BND && nbe < 0;
+      const bool out = side || bdr;  // n points out of the element
+      double n[DIM];
+#pragma unroll
+      for (int dd = 0; dd < DIM; ++dd) n[dd] = side ? met[dd] : (bdr ? -met[dd] : nl[dd]);
+      if constexpr (BND) {
+        if (bdr) {
+          const int b = -(nbe + 1), type = a.bc_type[b];
+          if (bc_wall_pressure(type, VISC) || bc_zero_flux(type, VISC)) {
+            const double pw = bc_zero_flux(type, VISC) ? 0.0 : slipwall_pstar<DIM>(g, qn[side], n);
+#pragma unroll
+            for (int dd = 0; dd < DIM; ++dd) rate[m][1 + dd] += B.iw[0] * (pw * n[dd]);
+            continue;
+          }
+          bc_exterior<DIM>(type, a.bc_data + (size_t)b * BC_STRIDE, n, qn[side]);
+        }
+      }
       Pt<double, DIM> own = end[side], oth;
       // momentum and energy again from LDS rather than held through the volume terms
 #pragma unroll
@@ -580,16 +605,23 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) k_
       if constexpr (SURF == 5) {
         // with VISC F* - 0.5 n.(Fv_L + Fv_R) (DGSEMIntegrator.hpp:261-316); the
         // own side's -0.5 n.Fv was folded into Vd by the gradient kernel
-        lift_llf_f64<DIM>(g, own, oth, n, side ? 1.0 : -1.0, side ? B.iw[0] : -B.iw[0], gn[side], rate[m]);
+        lift_llf_f64<DIM>(g, own, oth, n, out ? 1.0 : -1.0, out ? B.iw[0] : -B.iw[0], gn[side], rate[m]);
       } else {
         double F[NQ];
-        surface_flux<SURF, double, DIM>(g, side ? own : oth, side ? oth : own, n, F);
+        if constexpr (BND) {
+          Pt<double, DIM> pl, pr;
+          pt_select(out, own, oth, pl);
+          pt_select(out, oth, own, pr);
+          surface_flux<SURF, double, DIM>(g, pl, pr, n, F);
+        } else {
+          surface_flux<SURF, double, DIM>(g, side ? own : oth, side ? oth : own, n, F);
+        }
         if constexpr (VISC) {
 #pragma unroll
           for (int c = 0; c < NVD; ++c) F[1 + c] -= 0.5 * gn[side][c];
         }
 #pragma unroll
-        for (int c = 0; c < NQ; ++c) rate[m][c] += (side ? B.iw[0] : -B.iw[0]) * F[c];
+        for (int c = 0; c < NQ; ++c) rate[m][c] += (out ? B.iw[0] : -B.iw[0]) * F[c];
       }
     }
     // ---- the sums move to the next direction's lines
