@@ -13,17 +13,18 @@
 // it, and a workgroup is one wave without barriers.
 //
 // Memory bounds it: HBM (on 32^3 elements, p = 3, with viscous terms 506 MB a
-// launch, 98 us at the rate of a copy) and the vector memory path to it (TD busy
-// 80 % of the time), not the FP64 issue (35 %).  So own data moves in memory order, 512 consecutive
-// bytes a wave instruction, and changes to lines in LDS, neighbours along x
-// come from the wave's own LDS, and per-element values are loaded by
-// consecutive lanes once.  With a lane loading and storing its x-line's nodes
-// (32 bytes apart) and each element's values in all its lanes, an SSP-RK3 step
-// on 48^3 elements, p = 3, Ranocha/LLF with viscous terms took 1761 us, now
-// 1600; an Euler evaluation on 17 x 15 x 13 elements at p = 4 24.5 us, now 22.3.
-// On 32^3 elements the kernel takes 96 to 107 us, on different cards, for the
-// node form's 145 to 173, with 21 M vector instructions for 53 M, at 240
-// registers: two waves a SIMD (three spill and are slower).
+// launch, 98 us at the rate of a copy) and the vector memory path to it (TD
+// busy 80 % of the time), not the FP64 issue (35 %).  So own data moves in
+// memory order, 512 consecutive bytes a wave instruction, and changes to lines
+// in LDS, neighbours along x come from the wave's own LDS, and per-element
+// values are loaded by consecutive lanes once.  With a lane loading and storing
+// its x-line's nodes (32 bytes apart) and each element's values in all its
+// lanes, an SSP-RK3 step on 48^3 elements, p = 3, Ranocha/LLF with viscous terms
+// took 1761 us, now 1540 (k_ns_grad_line's share included); an Euler evaluation
+// on 17 x 15 x 13 elements at p = 4 24.5 us, now 22.3.  On 32^3 elements the
+// kernel takes 96 to 107 us, on different cards, for the node form's 145 to 173,
+// with 21 M vector instructions for 53 M, at 240 registers: two waves a SIMD
+// (three spill and are slower).
 #pragma once
 
 #include "rhs_kernels.hpp"
