@@ -715,12 +715,17 @@ __device__ __forceinline__ void entropy_state(const GasC<R> &g, const R *q, R *E
 // (grad p = (p/rho) (grad rho + p grad(-beta)), so grad p - (p/rho) grad rho
 // holds grad(-beta) alone).  Leaving it out drops two logarithms a state, a
 // fifth of the contractions, and the rounding of that cancellation.
+// Its logarithms made a state with rho <= 0 or p <= 0 NaN in FP32 (ln_pos does
+// not in FP64); with the central volume flux nothing else at an interior node
+// does, so the FP32 form says it here.
 template <typename R, int DIM>
 __device__ __forceinline__ void viscous_variables(const GasC<R> &g, const R *q, R *S) {
   const NodeThermo<R, DIM> t = node_thermo<R, DIM>(g, q);
+  R beta = t.beta;
+  if constexpr (sizeof(R) == sizeof(float)) beta = t.rho > R(0) && t.p > R(0) ? beta : R(__builtin_nanf(""));
 #pragma unroll
-  for (int d = 0; d < DIM; ++d) S[d] = t.beta * t.u[d];
-  S[DIM] = -t.beta;
+  for (int d = 0; d < DIM; ++d) S[d] = beta * t.u[d];
+  S[DIM] = -beta;
 }
 
 // One direction's velocity and temperature gradients from those variables'
