@@ -38,3 +38,19 @@ def test_mixed_navier_stokes_interior_node(dim, order, n, pairing, kind):
     nd = (order + 1) ** dim
     far = set(range(mesh.num_elements)) - {el} - {int(e) for e in mesh.face_neighbor.reshape(-1, 2 * dim)[el]}
     assert far and all(np.isfinite(got[:, e * nd:(e + 1) * nd]).all() for e in far)
+
+
+@pytest.mark.parametrize("dim,order,n", [(2, 3, (4, 4)), (2, 3, (129, 128)), (3, 2, (3, 3, 3)), (3, 2, (20, 19, 19)),
+                                         (3, 3, (3, 3, 3)), (3, 3, (13, 13, 13)), (3, 4, (3, 3, 3)), (3, 4, (13, 13, 13))])
+def test_infinite_pressure_reaches_the_face_flux(dim, order, n):
+    """Infinite energy at a face node: the sound speed there, the face's
+    dissipation and with it the density rates of both sides are not finite
+    (the node form on the small meshes, the line form on the others)."""
+    rt, mesh = make_case(dim, order, n, "ranocha_llf", blending=False)
+    U = smooth_state(mesh, order, rt.gamma, seed=order).reshape(dim + 2, -1)
+    el = mesh.num_elements // 2
+    low = int(mesh.face_neighbor.reshape(-1, 2 * dim)[el, 0])
+    own, other = _node(mesh, order, el, (0,) + (1,) * (dim - 1)), _node(mesh, order, low, (order,) + (1,) * (dim - 1))
+    U[-1, own] = np.inf
+    got = gpu_rhs(rt, mesh, U.reshape(-1))[0].reshape(dim + 2, -1)
+    assert not np.isfinite(got[0, [own, other]]).any(), got[:, [own, other]]

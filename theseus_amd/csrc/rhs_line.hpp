@@ -148,17 +148,18 @@ __device__ __forceinline__ void line_ranocha_f64(const GasC<double> &g, const Pt
 }
 
 // Square root of a normal x by Goldschmidt's iteration from the hardware
-// estimate, with a final remainder correction (within an ulp); 0 for 0, NaN
-// below.  10 instructions for the 20 of the correctly rounded form, which
-// also scales for subnormal arguments.
+// estimate, with a final remainder correction (within an ulp); 0 and infinity
+// themselves, NaN below.  10 instructions for the 20 of the correctly rounded
+// form, which also scales for subnormal arguments.
 __device__ __forceinline__ double sqrt_nr(double x) {
+  constexpr int kZeroOrInfinity = 1 << 5 | 1 << 6 | 1 << 9;  // -0, +0, +infinity of v_cmp_class
   const double y = __builtin_amdgcn_rsq(x);
   double g = x * y, h = 0.5 * y;
   const double r = fma(-h, g, 0.5);
   g = fma(g, r, g);
   h = fma(h, r, h);
   g = fma(fma(-g, g, x), h, g);
-  return x == 0.0 ? x : g;
+  return __builtin_amdgcn_class(x, kZeroOrInfinity) ? x : g;
 }
 
 // A face point's Lax-Friedrichs flux (LaxFriedrichsFlux.hpp:188-211) in FP64,
