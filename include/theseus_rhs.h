@@ -352,6 +352,9 @@ THESEUS_API int theseus_rhs_enable_kernel_timing(theseus_rhs *h, int capacity);
 /* Synchronises the recorded events; returns the mean duration in ms and the
  * number of timed launches of one kernel kind. */
 THESEUS_API int theseus_rhs_kernel_timing(theseus_rhs *h, int kind, double *mean_ms, int *count);
+/* *line = 1 if the handle's evaluations run that kind's line form (one lane
+ * per GLL line), 0 if its node form. */
+THESEUS_API int theseus_rhs_kernel_form(const theseus_rhs *h, int kind, int *line);
 
 /* ---- element orientation (the counterpart of MFEM's face orientations,
  * dgsem_cache_utilities.hpp:533-541, GetPermutedIndex) -------------------

@@ -67,6 +67,7 @@ EXPORTED_SYMBOLS = (
     "theseus_rhs_step_ssprk3_cfl",
     "theseus_rhs_enable_kernel_timing",
     "theseus_rhs_kernel_timing",
+    "theseus_rhs_kernel_form",
     "theseus_last_error",
     "theseus_pool_create",
     "theseus_pool_destroy",
@@ -218,6 +219,8 @@ def load(path: Path | str | None = None) -> C.CDLL:
     lib.theseus_rhs_enable_kernel_timing.restype = C.c_int
     lib.theseus_rhs_kernel_timing.argtypes = [C.c_void_p, C.c_int, C.POINTER(C.c_double), C.POINTER(C.c_int)]
     lib.theseus_rhs_kernel_timing.restype = C.c_int
+    lib.theseus_rhs_kernel_form.argtypes = [C.c_void_p, C.c_int, C.POINTER(C.c_int)]
+    lib.theseus_rhs_kernel_form.restype = C.c_int
     lib.theseus_rhs_integral_measures.argtypes = [C.c_void_p, C.c_void_p, C.POINTER(IntegralMeasures), C.c_void_p]
     lib.theseus_rhs_integral_measures.restype = C.c_int
     lib.theseus_rhs_integral_measures_baseline.argtypes = [C.c_void_p, C.POINTER(IntegralMeasures)]

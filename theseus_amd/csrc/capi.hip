@@ -1225,6 +1225,12 @@ int theseus_rhs_kernel_timing(theseus_rhs *h, int kind, double *mean_ms, int *co
   return THESEUS_OK;
 }
 
+int theseus_rhs_kernel_form(const theseus_rhs *h, int kind, int *line) {
+  if (!h || kind < 0 || kind > 1 || !line) return fail(THESEUS_ERR_INVALID_ARGUMENT, "bad arguments");
+  *line = kind == 0 ? h->line : h->grad_line;
+  return THESEUS_OK;
+}
+
 int theseus_rhs_destroy(theseus_rhs *h) {
   if (!h) return THESEUS_OK;
   release_events(h);

@@ -269,6 +269,12 @@ class RHSOperator:
         A.check(self._lib, self._lib.theseus_rhs_kernel_timing(self._h, int(kind), C.byref(ms), C.byref(n)))
         return float(ms.value), int(n.value)
 
+    def kernel_form(self, kind: int) -> str:
+        """"line" or "node": the form of kernel kind 0 or 1 the evaluations run."""
+        line = C.c_int()
+        A.check(self._lib, self._lib.theseus_rhs_kernel_form(self._h, int(kind), C.byref(line)))
+        return "line" if line.value else "node"
+
     def close(self) -> None:
         if getattr(self, "_h", None):
             self._lib.theseus_rhs_destroy(self._h)
