@@ -172,6 +172,14 @@ static void derivative_ops(int p, const std::vector<double> &x, const std::vecto
     b.w[i] = w[i];
     b.iw[i] = 1.0 / w[i];
   }
+  // The two-point fluxes of a line's end node sum to the flux times the
+  // off-diagonal sum of its row, +-1/w0 up to the rounding of the entries (3 to
+  // 4 units at p = 3 and 4); the face flux they nearly cancel with takes the same sum.
+  long double first = 0, last = 0;
+  for (int k = 1; k < Np; ++k) first += b.Dhat2[k];
+  for (int k = 0; k < Np - 1; ++k) last -= b.Dhat2[(Np - 1) * Np + k];
+  b.lift[0] = (double)first;
+  b.lift[1] = (double)last;
 }
 
 // Inverse of the 1-D Legendre Vandermonde V(i,a) = P_a(2 x_i - 1) on the

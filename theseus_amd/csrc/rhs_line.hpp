@@ -583,6 +583,7 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) k_
       const int nbe = side ? nhi : nlo;
       const bool bdr = BND && nbe < 0;
       const bool out = side || bdr;  // n points out of the element
+      const double lift = B.lift[side];
       double n[DIM];
 #pragma unroll
       for (int dd = 0; dd < DIM; ++dd) n[dd] = side ? met[dd] : (bdr ? -met[dd] : nl[dd]);
@@ -592,7 +593,7 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) k_
           if (bc_wall_pressure(type, VISC) || bc_zero_flux(type, VISC)) {
             const double pw = bc_zero_flux(type, VISC) ? 0.0 : slipwall_pstar<DIM>(g, qn[side], n);
 #pragma unroll
-            for (int dd = 0; dd < DIM; ++dd) rate[m][1 + dd] += B.iw[0] * (pw * n[dd]);
+            for (int dd = 0; dd < DIM; ++dd) rate[m][1 + dd] += lift * (pw * n[dd]);
             continue;
           }
           bc_exterior<DIM>(type, a.bc_data + (size_t)b * BC_STRIDE, n, qn[side]);
@@ -608,7 +609,7 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) k_
       if constexpr (SURF == 5) {
         // with VISC F* - 0.5 n.(Fv_L + Fv_R) (DGSEMIntegrator.hpp:261-316); the
         // own side's -0.5 n.Fv was folded into Vd by the gradient kernel
-        lift_llf_f64<DIM>(g, own, oth, n, out ? 1.0 : -1.0, out ? B.iw[0] : -B.iw[0], gn[side], rate[m]);
+        lift_llf_f64<DIM>(g, own, oth, n, out ? 1.0 : -1.0, out ? lift : -lift, gn[side], rate[m]);
       } else {
         double F[NQ];
         if constexpr (BND) {
@@ -624,7 +625,7 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) k_
           for (int c = 0; c < NVD; ++c) F[1 + c] -= 0.5 * gn[side][c];
         }
 #pragma unroll
-        for (int c = 0; c < NQ; ++c) rate[m][c] += (out ? B.iw[0] : -B.iw[0]) * F[c];
+        for (int c = 0; c < NQ; ++c) rate[m][c] += (out ? lift : -lift) * F[c];
       }
     }
     // ---- the sums move to the next direction's lines
