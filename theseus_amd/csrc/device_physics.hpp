@@ -722,7 +722,8 @@ template <typename R, int DIM>
 __device__ __forceinline__ void viscous_variables(const GasC<R> &g, const R *q, R *S) {
   const NodeThermo<R, DIM> t = node_thermo<R, DIM>(g, q);
   R beta = t.beta;
-  if constexpr (sizeof(R) == sizeof(float)) beta = t.rho > R(0) && t.p > R(0) ? beta : R(__builtin_nanf(""));
+  if constexpr (sizeof(R) == sizeof(float))
+    beta = t.rho * drcp(t.rho > R(0) && t.p > R(0) ? t.p : R(__builtin_nanf("")));  // a product, as t.beta, to be fused
 #pragma unroll
   for (int d = 0; d < DIM; ++d) S[d] = beta * t.u[d];
   S[DIM] = -beta;
