@@ -386,6 +386,12 @@ __global__ void __launch_bounds__(64) k_rates(unsigned long long *rates) {
     if (threadIdx.x == 0) rates[q] = (unsigned long long)__double_as_longlong(r[q]);
 }
 
+// Clears slots whose rates no kernel took (begin_estimate)
+__global__ void k_clear_rates(unsigned long long *rates) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < kRateWords) rates[i] = 0ull;
+}
+
 // Background pressure of the mixed mode: the pressure of the first node of
 // the state (one lane; a vector store).
 template <int DIM>
@@ -489,6 +495,27 @@ static double alpha_cut(double alpha_min) {
   return alpha_min > 0 && alpha_min < 1 ? std::log(1.0 / alpha_min - 1.0) + 1e-9 : HUGE_VAL;
 }
 
+// A stability estimate is a kernel that raises the rate slots and one that takes
+// and clears them.  If the second one's launch failed, the slots still hold the
+// first one's rates (`left`): the next estimate clears them before it starts, until
+// a clear has run (one recorded into a graph runs with the graph).
+static void begin_estimate(bool left, unsigned long long *rates, hipStream_t s) {
+  if (left) hipLaunchKernelGGL(k_clear_rates, dim3((kRateWords + 63) / 64), dim3(64), 0, s, rates);
+}
+static int end_estimate(bool &left, hipStream_t s) {
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess) {
+    left = true;
+    return fail(THESEUS_ERR_DEVICE, std::string("stability estimate: ") + hipGetErrorString(e));
+  }
+  if (left) {
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    HIP_TRY(hipStreamIsCapturing(s, &st));
+    left = st != hipStreamCaptureStatusNone;
+  }
+  return THESEUS_OK;
+}
+
 // Can the line forms (k_rhs_line, k_ns_grad_line) address ne elements' fields
 // and n.Fv rows with 32-bit byte offsets?
 static bool line_offsets(int ne, int ndof, int dim, int nfp) {
@@ -566,6 +593,7 @@ struct theseus_rhs {
   bool pref_set = false;
   double *d_stage[2] = {nullptr, nullptr};
   unsigned long long *d_rates = nullptr;  // d_words->rates
+  bool rates_left = false;            // begin_estimate
   double *d_meas = nullptr;           // integral measures: [nblocks][9] partials, then the 9 results
   double *d_ent = nullptr;            // entropy production: [nodes/256][2] partials, then the 2 results
   theseus_integral_measures diag0{};  // baseline: the first measures with nonzero mass
@@ -1322,8 +1350,9 @@ static int enqueue_ssprk3(theseus_rhs *h, double *u, double dt, const double *dt
   return enqueue_rhs(h, a, s);
 }
 
-// Launches the stability kernel; a kernel that takes its rates (take_rates) follows it.
+// Launches the stability kernel; a kernel that takes its rates (take_rates) and end_estimate follow it.
 static void enqueue_stability(theseus_rhs *h, const double *u, hipStream_t s) {
+  begin_estimate(h->rates_left, h->d_rates, s);
   StabArgs a;
   std::memset(&a, 0, sizeof(a));
   a.U = u;
@@ -1406,8 +1435,9 @@ int theseus_rhs_step_ssprk3_cfl(theseus_rhs *h, double *u, theseus_clock *clock,
   }
   enqueue_stability(h, ua, s);
   hipLaunchKernelGGL(k_clock, dim3(1), dim3(64), 0, s, clock, h->d_rates);
-  HIP_TRY(hipGetLastError());
-  const int rc = enqueue_ssprk3(h, ua, 0.0, &clock->dt_real, s);
+  int rc = end_estimate(h->rates_left, s);
+  if (rc) return rc;
+  rc = enqueue_ssprk3(h, ua, 0.0, &clock->dt_real, s);
   if (rc || !h->d_orient) return rc;
   return orient_pass(h, h->d_ual, u, false, s);
 }
@@ -1534,11 +1564,11 @@ int theseus_rhs_estimate_stability(theseus_rhs *h, const double *u, theseus_stab
   if (!h || !u || !out) return fail(THESEUS_ERR_INVALID_ARGUMENT, "null handle, vector or output");
   hipStream_t s = (hipStream_t)stream;
   const double *ua = u;
-  const int rc = aligned_input(h, u, &ua, s);
+  int rc = aligned_input(h, u, &ua, s);
   if (rc) return rc;
   enqueue_stability(h, ua, s);
   hipLaunchKernelGGL(k_rates, dim3(1), dim3(64), 0, s, h->d_rates);
-  HIP_TRY(hipGetLastError());
+  if ((rc = end_estimate(h->rates_left, s))) return rc;
   unsigned long long r[3];
   HIP_TRY(hipMemcpyAsync(r, h->d_rates, sizeof r, hipMemcpyDeviceToHost, s));
   HIP_TRY(hipStreamSynchronize(s));
@@ -1799,6 +1829,7 @@ struct theseus_pool {
   double *d_case_dt = nullptr, *d_case_pref = nullptr;
   SharedWords *d_words = nullptr;
   unsigned long long *d_rates = nullptr;  // d_words->rates
+  bool rates_left = false;   // begin_estimate
   double *d_meas = nullptr;  // integral measures: partials of the largest case, then the results
   std::vector<PoolCase> cases;
   std::vector<unsigned char> slot_used;  // per element slot
@@ -2331,11 +2362,12 @@ int theseus_pool_admit(theseus_pool *p, const theseus_case_desc *c, const double
   a.bc_data = p->d_bc_data;
   a.gas = p->gas;
   a.w0 = p->basis.w[0];
+  begin_estimate(p->rates_left, p->d_rates, s);
   p->sk->stability(a, (ne + p->sk->epb - 1) / p->sk->epb, s);
   hipLaunchKernelGGL(dim == 2 ? k_case_start<2> : k_case_start<3>, dim3(1), dim3(64), 0, s, p->d_rates, cfl,
                      p->d_case_dt + cid, p->d_U + off, p->Ntot, p->gas, p->d_case_pref + cid);
   hipLaunchKernelGGL(k_fill_i32, dim3((ne + 255) / 256), dim3(256), 0, s, p->d_elem_case + start, ne, cid);
-  HIP_TRY(hipGetLastError());
+  if ((rc = end_estimate(p->rates_left, s))) return rc;
   double dt = 0.0;
   if (dt_out) {
     // the caller asked for dt: wait for it, and refuse a case whose estimate is not usable
