@@ -82,8 +82,8 @@ def test_line_ends_at_rest(dim, n, order, pairing, visc):
     from theseus_amd.mesh import gll_nodes
     from theseus_amd.operator import MakeRHSOperator
 
-    if (dim, order, pairing, visc) == (3, 4, "hll", True):
-        pytest.skip("this pair's viscous form is not built in line form at order 4 in 3-D")
+    if dim == 3 and order > 2 and pairing == "hll" and visc:
+        pytest.skip("this pair's viscous form is not built in line form above order 2 in 3-D")
     flow = A.FLOW_NAVIER_STOKES if visc else A.FLOW_EULER
     rt, mesh = make_case(dim, order, n, pairing, flow=flow, blending=False)
     nd, Np = (order + 1) ** dim, order + 1

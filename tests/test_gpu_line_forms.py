@@ -70,34 +70,58 @@ def _moved(U, mesh, back):
     return np.ascontiguousarray(U.reshape(mesh.dim + 2, mesh.num_elements, -1)[:, back]).reshape(-1)
 
 
-@pytest.mark.parametrize("dim,n,order,pairing,visc,forms", [
-    (3, (16, 16, 8), 3, "ranocha_llf", False, ("line", "node")),   # 512 waves of 4 elements
-    (3, (16, 16, 8), 3, "ranocha_llf", True, ("line", "line")),
-    (3, (127, 4, 4), 3, "ranocha_llf", True, ("node", "node")),    # 508
-    (3, (16, 16, 8), 3, "hll", True, ("node", "line")),            # this pair from 1024
-    (3, (16, 16, 16), 3, "hll", True, ("line", "line")),
-    (3, (8, 8, 8), 4, "ranocha_llf", True, ("node", "node")),      # 256 of 2
-    (3, (16, 16, 8), 4, "ranocha_llf", True, ("line", "line")),    # 1024
-    (3, (16, 16, 8), 4, "hll", False, ("node", "node")),           # from 2048
-    (3, (16, 16, 16), 4, "hll", False, ("line", "node")),
-    (3, (16, 16, 16), 4, "hll", True, ("node", "line")),           # not built
-    (3, (24, 24, 24), 3, "pirozzoli", False, ("node", "node")),
-    (2, (128, 128), 3, "chandrashekar_roe", False, ("line", "node")),  # 1024 of 16
-    (2, (128, 127), 3, "chandrashekar_roe", True, ("node", "line")),
-    (2, (64, 64), 1, "ranocha_llf", True, ("node", "node")),
+@pytest.mark.parametrize("dim,n,order,pairing,visc,blending,forms", [
+    (3, (16, 16, 12), 3, "ranocha_llf", False, True, ("line", "node")),   # 768 waves of 4 elements
+    (3, (16, 16, 12), 3, "ranocha_llf", True, True, ("line", "line")),
+    (3, (17, 15, 12), 3, "ranocha_llf", True, True, ("node", "line")),    # 765
+    (3, (127, 4, 4), 3, "llf", True, True, ("node", "node")),             # 508
+    (3, (16, 16, 8), 3, "llf", True, True, ("line", "line")),             # 512
+    (3, (16, 16, 8), 3, "hll", False, True, ("line", "node")),
+    (3, (16, 16, 32), 3, "hll", True, True, ("node", "line")),            # not built
+    (3, (16, 15, 24), 3, "chandrashekar", False, False, ("node", "node")),  # 1440 of 1536
+    (3, (16, 16, 24), 3, "chandrashekar", False, True, ("line", "node")),
+    (3, (16, 32, 31), 3, "chandrashekar_roe", True, True, ("node", "line")),  # 3968 of 4096
+    (3, (16, 32, 32), 3, "chandrashekar_roe", True, False, ("line", "line")),
+    (3, (8, 8, 8), 4, "ranocha_llf", True, True, ("node", "node")),       # 256 of 2
+    (3, (16, 16, 8), 4, "ranocha_llf", True, True, ("node", "line")),     # 1024
+    (3, (16, 16, 12), 4, "ranocha_llf", True, True, ("line", "line")),    # 1536
+    (3, (16, 16, 12), 4, "hll", False, True, ("node", "node")),           # from 2048
+    (3, (16, 16, 16), 4, "hll", False, True, ("line", "node")),
+    (3, (16, 16, 64), 4, "llf", True, True, ("node", "line")),            # not built
+    (3, (24, 24, 24), 3, "pirozzoli", False, True, ("node", "node")),
+    (2, (128, 128), 3, "chandrashekar_roe", False, False, ("line", "node")),  # 1024 of 16
+    (2, (128, 128), 3, "chandrashekar_roe", False, True, ("node", "node")),   # with blending from 6144
+    (2, (256, 384), 3, "chandrashekar_roe", False, True, ("line", "node")),
+    (2, (128, 191), 3, "ranocha_llf", False, True, ("node", "node")),         # 1528 of 1536
+    (2, (128, 192), 3, "ranocha_llf", False, True, ("line", "node")),
+    (2, (128, 128), 3, "hll", True, True, ("line", "line")),
+    (2, (64, 64), 1, "ranocha_llf", True, True, ("node", "node")),
 ])
-def test_forms(dim, n, order, pairing, visc, forms):
-    rt, mesh = make_case(dim, order, n, pairing, flow=_flow(visc))
+def test_forms(dim, n, order, pairing, visc, blending, forms):
+    rt, mesh = make_case(dim, order, n, pairing, flow=_flow(visc), blending=blending)
     op, got = _operator(rt, mesh)
     op.close()
     assert got == forms
 
 
+@pytest.mark.parametrize("dim,n,order,pairing,form", [
+    (3, (16, 16, 8), 3, "hll", "node"), (3, (16, 16, 12), 3, "hll", "line"),                    # from 768 waves, periodic 512
+    (3, (16, 16, 16), 3, "ranocha", "node"), (3, (16, 16, 24), 3, "ranocha", "line"),           # from 1536, periodic 1024
+    (3, (16, 16, 11), 3, "ranocha_llf", "node"), (3, (17, 16, 16), 4, "llf", "node"),           # not built
+])
+def test_forms_with_boundaries(dim, n, order, pairing, form):
+    rt, mesh = _bc_case(dim, order, n, pairing, A.FLOW_EULER, "euler", blending=True)
+    op, got = _operator(rt, mesh)
+    op.close()
+    assert got == (form, "node")
+
+
 @pytest.mark.parametrize("kind", ["sheared", "graded", "own"])
 @pytest.mark.parametrize("noise", ["short", "far"])
 @pytest.mark.parametrize("dim,n,order,pairing,visc", [
-    (2, (147, 147), 2, "chandrashekar_roe", True), (2, (129, 128), 3, "ranocha_llf", True), (2, (111, 111), 4, "ranocha", False),
-    (3, (20, 19, 19), 2, "ranocha_llf", True), (3, (13, 13, 13), 3, "ranocha_llf", False), (3, (17, 15, 17), 3, "ranocha_llf", True),
+    (2, (147, 147), 2, "chandrashekar_roe", True), (2, (160, 154), 3, "ranocha_llf", True), (2, (193, 192), 4, "ranocha", False),
+    (3, (20, 19, 19), 2, "ranocha_llf", True), (3, (16, 16, 13), 3, "ranocha_llf", False), (3, (17, 15, 17), 3, "ranocha_llf", True),
+    (3, (24, 23, 12), 3, "chandrashekar", False), (3, (32, 32, 17), 3, "chandrashekar_roe", True),
     (3, (17, 16, 17), 3, "roe", True), (3, (17, 15, 17), 4, "ranocha_llf", True), (3, (17, 16, 17), 4, "hll", False),
 ])
 def test_metrics_and_numbering(oracle, dim, n, order, pairing, visc, noise, kind):
@@ -117,7 +141,7 @@ def test_metrics_and_numbering(oracle, dim, n, order, pairing, visc, noise, kind
 @pytest.mark.parametrize("sides", ["euler", "no_slip"])
 @pytest.mark.parametrize("noise", ["short", "far"])
 @pytest.mark.parametrize("dim,n,order,pairing", [
-    (2, (129, 128), 3, "ranocha_llf"), (2, (147, 147), 2, "chandrashekar"), (3, (17, 17, 17), 3, "hll"),
+    (2, (160, 154), 3, "ranocha_llf"), (2, (147, 147), 2, "chandrashekar"), (3, (17, 17, 17), 3, "hll"),
     (3, (17, 16, 16), 4, "ranocha_llf"), (3, (17, 16, 16), 4, "ranocha"), (3, (17, 16, 17), 4, "hll"),
 ])
 def test_metrics_and_boundaries(oracle, dim, n, order, pairing, noise, sides, kind):
@@ -138,7 +162,7 @@ def test_stored_frames(visc):
     results, bit for bit."""
     from theseus_amd.meshio import to_aligned, to_storage
 
-    rt, box = make_case(3, 3, (13, 13, 13), "ranocha_llf", flow=_flow(visc), blending=True)
+    rt, box = make_case(3, 3, (15, 15, 14), "ranocha_llf", flow=_flow(visc), blending=True)
     mesh = SimpleNamespace(**{k: getattr(box, k) for k in ("dim", "num_elements", "face_neighbor", "bc_type", "elem_jac",
                                                            "elem_adj", "lower", "upper")})
     mesh.elem_orient = np.random.default_rng(5).integers(0, 48, size=box.num_elements).astype(np.uint8)
@@ -153,7 +177,7 @@ def test_stored_frames(visc):
     np.testing.assert_array_equal(got, ref)
 
 
-@pytest.mark.parametrize("dim,n,order,visc", [(2, (129, 128), 3, True), (3, (13, 13, 13), 3, True), (3, (17, 15, 17), 4, False)])
+@pytest.mark.parametrize("dim,n,order,visc", [(2, (160, 154), 3, True), (3, (15, 15, 14), 3, True), (3, (17, 15, 17), 4, False)])
 def test_device_clock_and_graph(dim, n, order, visc):
     """Steps of the length the device chooses equal steps given that length, and
     recorded steps equal eager ones, bit for bit, on every replay with eager

@@ -523,10 +523,10 @@ static bool line_offsets(int ne, int ndof, int dim, int nfp) {
 }
 
 // Does the fused kernel run in its line form on ne elements?  Where it is
-// built, on enough waves to fill the chip (line_min_waves).
-static bool line_form(const FluxKernels *fk, bool ns, bool boundary, int ne) {
+// built, on enough waves (line_min_waves).
+static bool line_form(const FluxKernels *fk, bool ns, bool boundary, bool blending, int ne) {
   if (!fk || !(ns ? (boundary ? nullptr : fk->ns_line) : fk->euler_line[boundary])) return false;
-  return (ne + fk->line_epw - 1) / fk->line_epw >= (ns ? fk->ns_line_min : fk->euler_line_min);
+  return (ne + fk->line_epw - 1) / fk->line_epw >= (ns ? fk->ns_line_min[blending] : fk->euler_line_min[boundary][blending]);
 }
 
 // Does the gradient pass?  Where it is built, on enough waves
@@ -1089,7 +1089,7 @@ static int create_impl(const theseus_case_desc *desc, const theseus_lte_table *l
   h->pm = d.precision == THESEUS_PRECISION_MIXED ? 1 : 0;
   if (!lk && h->pm == 0 && line_offsets(ne, h->ndof, dim, h->nfp)) {
     const bool ns = d.flow_model == THESEUS_FLOW_NAVIER_STOKES;
-    h->line = line_form(fk, ns, has_boundary, ne);
+    h->line = line_form(fk, ns, has_boundary, d.blending != 0, ne);
     h->grad_line = ns && !has_boundary && grad_line_form(sk, d);
   }
   h->adv_scale = advection_scale(d.order);

@@ -24,9 +24,9 @@ struct FluxKernels {
   RHSLaunch euler[2][2] = {};  // fused volume + face
   RHSLaunch ns[2][2] = {};     // Navier-Stokes pass 2
   // the FP64 line form (k_rhs_line) on meshes without ([0]) and with boundary faces (Euler), and the
-  // fewest workgroups (waves of line_epw elements) it is used from; null where it is not built
+  // fewest workgroups (waves of line_epw elements) it is used from, by [boundary][blending]; null where it is not built
   RHSLaunch euler_line[2] = {}, ns_line = nullptr;
-  int euler_line_min = 0, ns_line_min = 0;
+  int euler_line_min[2][2] = {}, ns_line_min[2] = {};
   int line_epw = 0;
 };
 
@@ -105,44 +105,70 @@ void launch_measures(const MeasArgs &a, int nb, hipStream_t s) {
   hipLaunchKernelGGL((k_measures<DIM, P>), dim3(nb), dim3(Shape<DIM, P>::TPB), 0, s, a);
 }
 
-// From how many waves on the line form (k_rhs_line) is the faster one, 0 where
+// From how many waves on the line form (k_rhs_line) is not the slower one, 0 where
 // it is not built.  It issues 0.4 to 0.6 of the node form's instructions but
-// runs Np nodes in each lane's chain, so it needs waves to hide latency: one
-// per SIMD (1024 waves) is about where it begins to win.  Ratio of the times,
-// node / line form, of a whole evaluation (with NS also of the gradient pass)
-// at 512, 1024, 2048 and 4096 waves:
-//   3-D p = 3  Ranocha/LLF Euler 1.27 1.46 1.81 1.75, NS 1.15 1.25 1.44 1.42;
-//              central/HLL Euler 1.13 1.28 1.58 1.52, NS 0.95 0.99 1.19 1.21;
-//              Chandrashekar/Roe Euler 1.10 1.52 1.49 1.44, NS 0.90 1.10 1.27 1.17
-//   3-D p = 2  Ranocha/LLF Euler 1.14 1.49 1.64 1.56, NS 1.12 1.29 1.35 1.21;
-//              Chandrashekar/Roe Euler 1.06 1.49 1.49 1.38, NS 1.05 1.32 1.38 1.23
-//   2-D p = 3  Ranocha/LLF Euler 1.01 1.19 1.44 1.44, NS 0.97 1.12 1.25 1.29;
-//              Chandrashekar/Roe Euler 0.83 1.04 1.26 1.29, NS 0.91 1.04 1.21 1.21
-// Order 4 in 3-D (two elements in 50 of 64 lanes, five nodes a lane) needs the
-// registers: Ranocha/LLF Euler 1.04 1.26 1.62 1.57, NS 0.91 1.04 1.31 1.30,
-// Ranocha/Ranocha NS 0.76 0.93 1.17 1.16, central/LLF NS 0.79 0.95 1.14 1.06,
-// central/HLL Euler 0.78 0.89 1.11 1.02, but NS 0.61 0.75 0.93 0.88 and
-// Chandrashekar's Euler 0.62 0.78 1.02 0.96, where it is left out, as it is for
-// Chandrashekar's 2-D NS at p = 4 (0.68 0.91 0.97 1.22) and Pirozzoli's (3-D
-// p = 3 Euler 0.83 0.96 1.06 1.02, NS 0.60 0.76 0.89 0.84).
-// In the mixed mode, whose node form is shorter and whose line form held three
-// sets of sums, the ratios at p = 3 were 1.03 1.06 1.33 1.14 for Euler and 0.96
-// 0.98 1.14 1.02 for NS, at p = 4 0.81 0.89 1.15 1.09 and 0.82 0.96 1.10 1.04,
-// and a pool's results would depend on its launch range: FP64 only.
-// With boundary faces (Euler; at 1024, 2048 and 4096 waves): 2-D Ranocha/LLF
-// p = 3 1.07 1.27 1.18, p = 4 1.14 1.25 1.47, central/HLL p = 4 1.26 1.25 1.42;
-// 3-D Ranocha/LLF p = 3 1.43 1.74 1.68, central/HLL p = 2 1.01 1.41 1.26; but
-// Chandrashekar's 2-D p = 3 1.01 1.06 0.99 and p = 4 0.98 0.96 1.13, left out,
-// as are central/LLF and central/Roe in 3-D at p = 4 (332 and 424 B of scratch).
+// runs Np nodes in each lane's chain, so it needs waves to hide latency, and a
+// wave that holds one blended element makes the subcell pass for all of its
+// elements (2-D p = 3: 16).  At two waves a SIMD its time is a staircase of 1024
+// (up to 1024 waves one each) and 2048 waves: the ratios dip just above them.
+// Ratio of the times, node / line form, of a whole evaluation (with NS the
+// gradient pass by its own rule), smooth state / state with shocks (blended
+// elements along two lines or three planes, 1 to 2 % and 10 to 25 % of all):
+//   waves              768        1024        1152        1536        2304        4096
+//   2-D p = 3, periodic
+//     Ranocha/LLF   1.18/0.91  1.28/1.14  1.28/0.90  1.38/1.00  1.44/1.29  1.38/1.13
+//     central/HLL   1.12/1.01  1.23/1.25  1.16/1.07  1.35/1.09  1.24/1.09  1.42/1.12
+//     Ch'kar/Roe    1.10/0.85  1.23/1.12  1.09/0.79  1.17/0.92  1.15/0.94  1.38/0.98
+//     Ranocha       1.06/0.82  1.18/1.06  1.08/0.79  1.17/0.89  1.14/0.92  1.33/0.97, at 6144 1.39/1.02
+//   2-D p = 4  Ranocha  1.43/0.91  1.51/0.93  1.31/0.95  1.53/0.85  1.47/0.98  1.78/1.18, at 3072 1.69/1.07
+//     central/HLL, outflow boundary 1.26/1.10  1.40/1.21  1.23/1.08  1.35/1.08  1.35/1.17  1.61/1.30
+//   3-D p = 2  Ranocha/LLF  1.22/1.19  1.37/1.35  1.12/1.10  1.44/1.26  1.29/1.31  1.55/1.30, at 512 0.91/0.91
+//     Ch'kar/Roe    1.04/1.17  1.27/1.31  0.95/1.05  1.25/1.15  1.18/1.22  1.48/1.25
+//   3-D p = 3
+//     Ranocha/LLF   1.20/1.01  1.25/1.08  1.10/1.02  1.33/1.10  1.34/1.10  1.65/1.35, at 512 0.99/0.78
+//       boundary    1.19/1.01  1.16/1.08  1.06/1.03  1.32/1.09  1.28/1.05  1.62/1.32, at 512 0.94/0.78
+//       NS          1.12/1.01  1.12/1.01  1.04/0.99  1.15/1.07  1.15/1.09  1.30/1.21, at 512 0.95/0.80
+//     central/HLL   1.28/1.21  1.31/1.30  1.23/1.13  1.47/1.33  1.34/1.19  1.54/1.40, at 512 1.05/0.96
+//       boundary    1.13/1.11  1.14/1.17  1.09/1.04  1.27/1.22  1.18/1.09  1.36/1.30, at 512 0.91/0.90
+//       NS          0.94/0.97  0.93/0.99  0.93/0.95  1.01/1.02  0.94/0.97  1.06/1.11, at 8192 0.87/0.93: not built
+//     Ch'kar/Roe    0.85/0.87  1.16/1.18  0.89/0.94  1.05/1.04  1.09/1.04  1.47/1.29
+//       NS          0.71/0.77  0.87/0.98  0.79/0.87  0.86/0.93  0.86/0.90  1.06/1.07, at 8192 1.03/1.07
+//     Ranocha       0.99/0.85  1.39/1.17  1.02/0.95  1.25/1.06  1.26/1.02  1.61/1.29
+//       boundary    0.94/0.84  1.30/1.13  0.98/0.93  1.20/1.02  1.21/0.98  1.54/1.23
+//   3-D p = 4 (two elements in 50 of 64 lanes, five nodes a lane)
+//     Ranocha/LLF   1.06/0.88  1.08/0.90  0.93/0.93  1.10/1.03  1.14/1.10  1.37/1.15
+//       NS          0.76/0.75  0.95/0.87  0.90/0.91  1.00/0.96  1.00/0.95  1.15/1.05
+//     central/HLL   0.96/0.93  0.93/0.93  0.88/0.91  1.01/0.99  0.96/0.96  1.11/1.05, at 2048 1.18/1.19
+//     Ranocha NS    0.62/0.60  0.95/0.89  0.82/0.83  0.88/0.90  0.90/0.89  1.09/0.97
+//     central/LLF NS 0.81/0.79 0.90/0.93  0.91/0.91  0.99/0.95  0.86/0.87  1.00/1.01, at 8192 0.88/0.93: not built
+// The minimum is where both stay above 0.95, the runs' own spread, from there on;
+// without blending the first alone, which in 2-D is lower.  Left out as well, from
+// ratios at 512, 1024, 2048 and 4096 waves without shocks: 3-D p = 4 central/HLL NS
+// (0.61 0.75 0.93 0.88) and Chandrashekar (Euler 0.62 0.78 1.02 0.96), 2-D p = 4
+// Chandrashekar NS (0.68 0.91 0.97 1.22), Pirozzoli (3-D p = 3 Euler 0.83 0.96 1.06 1.02,
+// NS 0.60 0.76 0.89 0.84); with boundary faces at 1024, 2048 and 4096, 2-D
+// Chandrashekar p = 3 (1.01 1.06 0.99) and p = 4 (0.98 0.96 1.13); and 3-D p = 4
+// central/LLF and central/Roe with boundary faces (332 and 424 B of scratch).
+// Mixed mode: not built.  Measured only with lanes that load their own line (before
+// the state moved in memory order), p = 3, waves as above: Euler 1.03 1.06 1.33
+// 1.14, NS 0.96 0.98 1.14 1.02; p = 4 0.81 0.89 1.15 1.09 and 0.82 0.96 1.10 1.04.
 template <int DIM, int P, int VOL, int SURF>
-constexpr int line_min_waves(bool visc, bool boundary = false) {
+constexpr int line_min_waves(bool visc, bool boundary, bool blending) {
   if (P < 2 || P > 4 || VOL == 3) return 0;
-  if (DIM == 3 && P == 4) {
-    if (VOL == 1 || (VOL == 0 && (visc ? SURF != 5 : boundary && SURF != 4))) return 0;
-    return VOL == 2 && (!visc || SURF == 5) ? 1024 : 2048;
+  const bool costly = VOL == 1 || SURF == 1;  // two-point fluxes with logarithms at the faces or divisions in the volume
+  if (DIM == 2) {
+    if (VOL == 1 && ((P == 4 && visc) || (P >= 3 && boundary))) return 0;
+    if (blending && P == 3) return costly ? 6144 : (VOL == 0 && SURF != 3 ? 1024 : 1536);
+    return blending && P == 4 && costly ? 3072 : 1024;
   }
-  if (DIM == 2 && VOL == 1 && ((P == 4 && visc) || (P >= 3 && boundary))) return 0;
-  return DIM == 3 && (SURF == 5 || (P == 3 && !visc)) ? 512 : 1024;
+  if (P == 2) return costly ? 1536 : (SURF == 5 ? 768 : 1024);
+  if (P == 3) {
+    if (visc) return VOL == 1 ? 4096 : SURF == 1 ? 1536 : SURF == 4 ? 0 : SURF == 3 ? 1024 : VOL == 2 ? 768 : 512;
+    if (VOL == 1 || (SURF == 1 && boundary)) return 1536;
+    return SURF == 1 ? 1024 : (boundary || VOL == 2 ? 768 : 512);
+  }
+  if (VOL == 1 || (VOL == 0 && (visc || (boundary && SURF != 4)))) return 0;
+  return VOL == 2 && SURF == 5 ? 1536 : (visc ? 4096 : 2048);
 }
 
 template <int DIM, int P, int VOL, int SURF, bool VISC, bool BND = false>
@@ -154,17 +180,15 @@ template <int DIM, int VOL, int SURF, int P>
 struct FluxRegistrar {
   FluxRegistrar() {
     FluxKernels k;
-    if constexpr (line_min_waves<DIM, P, VOL, SURF>(false) > 0) {
-      k.euler_line[0] = &launch_rhs_line<DIM, P, VOL, SURF, false>;
-      if constexpr (line_min_waves<DIM, P, VOL, SURF>(false, true) > 0)
-        k.euler_line[1] = &launch_rhs_line<DIM, P, VOL, SURF, false, true>;
-      k.euler_line_min = line_min_waves<DIM, P, VOL, SURF>(false);
-      k.line_epw = LineShape<DIM, P>::EPW;
+    constexpr auto min_waves = &line_min_waves<DIM, P, VOL, SURF>;
+    if constexpr (min_waves(false, false, false) > 0) k.euler_line[0] = &launch_rhs_line<DIM, P, VOL, SURF, false>;
+    if constexpr (min_waves(false, true, false) > 0) k.euler_line[1] = &launch_rhs_line<DIM, P, VOL, SURF, false, true>;
+    if constexpr (min_waves(true, false, false) > 0) k.ns_line = &launch_rhs_line<DIM, P, VOL, SURF, true>;
+    for (int blending = 0; blending < 2; ++blending) {
+      for (int boundary = 0; boundary < 2; ++boundary) k.euler_line_min[boundary][blending] = min_waves(false, boundary, blending);
+      k.ns_line_min[blending] = min_waves(true, false, blending);
     }
-    if constexpr (line_min_waves<DIM, P, VOL, SURF>(true) > 0) {
-      k.ns_line = &launch_rhs_line<DIM, P, VOL, SURF, true>;
-      k.ns_line_min = line_min_waves<DIM, P, VOL, SURF>(true);
-    }
+    if constexpr (P >= 2 && P <= 4) k.line_epw = LineShape<DIM, P>::EPW;
     k.euler[0][0] = &launch_rhs<double, DIM, P, VOL, SURF, false>;
     k.ns[0][0] = &launch_rhs<double, DIM, P, VOL, SURF, true>;
     k.euler[1][0] = &launch_rhs<float, DIM, P, VOL, SURF, false>;
