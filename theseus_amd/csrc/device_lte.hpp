@@ -180,27 +180,6 @@ __device__ __forceinline__ R evaluate(const Cell<R> &c, R xi, R eta) {
   return r / (cscale<DR>(c.wr) * cscale<DT>(c.wt));
 }
 
-template <int AXIS, int DR = 0, int DT = 0, typename R>
-__device__ __forceinline__ R divided(const Cell<R> &c, R xi1, R eta1, R xi2, R eta2) {
-  R r = 0;
-#pragma unroll
-  for (int i = 0; i < 2; ++i) {
-    const R rv = AXIS == 0 ? dpbasis<DR>(i, xi1, xi2) : pbasis<DR>(i, xi1);
-    const R rs = AXIS == 0 ? dsbasis<DR>(i, xi1, xi2) : sbasis<DR>(i, xi1);
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      const R tv = AXIS == 1 ? dpbasis<DT>(j, eta1, eta2) : pbasis<DT>(j, eta1);
-      const R ts = AXIS == 1 ? dsbasis<DT>(j, eta1, eta2) : sbasis<DT>(j, eta1);
-      const int o = i + j * c.stride;
-      r += c.H[o] * rv * tv;
-      r += (c.H[c.plane + o] * c.wr) * rs * tv;
-      r += (c.H[2 * c.plane + o] * c.wt) * rv * ts;
-      r += (c.H[3 * c.plane + o] * c.wr * c.wt) * rs * ts;
-    }
-  }
-  return r / (cscale<DR>(c.wr) * cscale<DT>(c.wt) * (AXIS == 0 ? c.wr : c.wt));
-}
-
 template <typename R = double>
 struct Eval {
   Cell<R> cell;
@@ -213,9 +192,6 @@ struct Eval {
   __device__ R energy() const { return H() - T * H<0, 1>(); }
   __device__ R gibbs() const { return H() + rho * H<1, 0>(); }
   __device__ R p_rho() const { return 2 * rho * H<1, 0>() + rho * rho * H<2, 0>(); }
-  __device__ R p_T() const { return rho * rho * H<1, 1>(); }
-  __device__ R g_rho() const { return 2 * H<1, 0>() + rho * H<2, 0>(); }
-  __device__ R g_T() const { return H<0, 1>() + rho * H<1, 1>(); }
   __device__ R cv() const { return -T * H<0, 2>(); }
   __device__ R cp() const {  // LTEHelmholtzEOS.hpp:76-80
     const R m = H<1, 1>();
@@ -349,9 +325,10 @@ __device__ __forceinline__ const R *cells_of(const View &v) {
   else return v.cells32;
 }
 
-// n / d with y the correctly rounded 1 / d: in FP64 the quotient estimate
-// n y corrected by its exact remainder, which rounds to the IEEE quotient in
-// three instructions instead of a division's eleven; FP32 divides.
+// n / d with y the correctly rounded 1 / d (Markstein's division by a known
+// reciprocal): in FP64 the quotient estimate n y corrected by its remainder,
+// which rounds as the IEEE quotient in three instructions instead of a
+// division's eleven; FP32 divides.
 template <typename R>
 __device__ __forceinline__ R div_by(R n, R d, R y) {
   if constexpr (sizeof(R) == sizeof(double)) {
@@ -385,8 +362,11 @@ __device__ __forceinline__ R pair_pressure(const PairNode<R> &s) {
 }
 
 // Products of a cell's coefficients with one rho basis (value side 0, 1,
-// slope side 0, 1), and their sum with one T basis: together evaluate()'s or
-// divided()'s operations in their order, the products shared by the T bases.
+// slope side 0, 1), and their sum with one T basis: evaluate()'s operations in
+// their order, the products shared by the T bases.  With the divided
+// differences of one direction's bases between two points (dbasis4) in place
+// of its bases, and divided by that direction's width once more, the sum is
+// the divided difference of the interpolant along it.
 template <typename R>
 struct Basis4 {
   R v0, v1, s0, s1;

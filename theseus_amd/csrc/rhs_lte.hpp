@@ -346,13 +346,8 @@ __global__ void __launch_bounds__((Shape<DIM, P>::TPB)) k_rhs_lte(RHSArgs a) {
 // three with the cell coefficients read twice and half the products live
 // (124 B) 230 us, the same as that form at two.
 template <typename R, int DIM, int P, bool VISC>
-struct LteecWaves {
-  static constexpr int value = 2;
-};
-
-template <typename R, int DIM, int P, bool VISC>
 __global__ void __launch_bounds__((Shape<DIM, P>::TPB))
-__attribute__((amdgpu_waves_per_eu(LteecWaves<R, DIM, P, VISC>::value))) k_rhs_lteec(RHSArgs a) {
+__attribute__((amdgpu_waves_per_eu(2))) k_rhs_lteec(RHSArgs a) {
   using S = Shape<DIM, P>;
   using VP = VolPlan<DIM, P, 0>;
   using SX = StagedIndex<S::Np, S::NDOF>;
