@@ -590,7 +590,7 @@ enum NodeOut { NODE_T = 0, NODE_LTEEC = 1, NODE_PC = 2 };
 // own, in its order.  The node values follow in the same kernel, where the
 // cell's record is at hand.  Latency of the dependent lookups (state, bucket,
 // inverse table, bucket, record) at 4 to 5 waves per SIMD bounds it.  At 24^3
-// elements, p = 3 (884,736 nodes): 46 us with LTEEC's values, 44 us with the
+// elements, p = 3 (884,736 nodes): 41 us with LTEEC's values, 42 us with the
 // other pairs', against 72 us for the recovery alone with both cells bisected
 // in every iteration and 39 (22) us for the values in a pass of their own.
 template <int DIM, int OUT, typename R = double>

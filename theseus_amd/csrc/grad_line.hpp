@@ -10,11 +10,12 @@
 // On 32^3 elements, p = 3, in FP64 it takes 70 us for the node form's 90, with
 // 11.4 M vector instructions for 28.9 M; its 300 MB of HBM traffic (133 read, 168
 // written) at the rate of a copy are 58 us.  The vector memory path is the bound
-// (TD busy 75 % of the time), with two waves a SIMD (220 registers; three spill).  On 48^3 elements
-// a step takes 1636 us for 1840 with the node form.  The mixed mode keeps the
-// node form: in FP32 this one took 47 us for 58, but folding the face lift into
-// the line's operator rounds the heat flux differently, up to 2.5e-8 of the
-// energy a step.
+// (TD busy 75 % of the time), with two waves a SIMD (220 registers; three spill).  Before k_rhs_line
+// moved in memory order a step on 48^3 elements took 1636 us with it and 1840 with
+// the node form.  The mixed mode keeps the node form: in FP32 this one took 47 us
+// for 58, but folding the face lift into the line's operator moved the outputs
+// by up to 2.5e-8 of the energy in two steps, and whether that is nearer to or
+// further from 64 bits was not measured.
 #pragma once
 
 #include "rhs_line.hpp"

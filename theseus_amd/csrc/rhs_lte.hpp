@@ -336,15 +336,16 @@ __global__ void __launch_bounds__((Shape<DIM, P>::TPB)) k_rhs_lte(RHSArgs a) {
 // pair evaluates only what depends on both endpoints (thermodynamic_means).
 // Bound by FP64 issue: 861 vector instructions a pair, none of which may be
 // contracted (device_lte.hpp), 72.7 M per launch at 24^3 elements, p = 3,
-// which issue in 145 us at the 2.0 GHz the card holds there.  Measured at that size: 218 us
-// (RHS 234 us with the node pass) against 926 us (964 us) when each pair
-// evaluated both endpoints and the two gradients separately, at one wave per
-// SIMD with 494 registers.
+// which issue in 145 us at the 2.0 GHz the card holds there.  Measured at that size:
+// 200 to 267 us, 241 on average, in the trace of the bench's steps, and 240 us for a
+// repeated evaluation with k_lte_nodes' 41, against 926 (969 with both passes) when
+// each pair evaluated both endpoints and the two gradients separately, at one
+// wave per SIMD with 494 registers.
 //
-// Occupancy asked of the register allocator: 2 waves per SIMD (256 registers,
-// no scratch in FP64).  Three (168 registers, 240 B of scratch per lane) took 282 us;
-// three with the cell coefficients read twice and half the products live
-// (124 B) 230 us, the same as that form at two.
+// Occupancy asked of the register allocator: 2 waves per SIMD (256 registers; no
+// scratch but 12 B in the FP64 Euler form of 3-D p = 3).  Three (168 registers, 240 B
+// of scratch per lane) took 282 us for 218; three with the cell coefficients read
+// twice and half the products live (124 B) 230 us, the same as that form at two.
 template <typename R, int DIM, int P, bool VISC>
 __global__ void __launch_bounds__((Shape<DIM, P>::TPB))
 __attribute__((amdgpu_waves_per_eu(2))) k_rhs_lteec(RHSArgs a) {
