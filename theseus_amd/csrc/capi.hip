@@ -101,10 +101,11 @@ const ShapeKernels *find_shape(int dim, int p) {
 
 // GLL nodes and weights on [0,1]: endpoints and the roots of P'_p, by Newton
 // iteration in long double, symmetrised (x_{p-i} = 1 - x_i).
-static void gll01(int p, std::vector<double> &x, std::vector<double> &w) {
+static void gll01(int p, std::vector<double> &x, std::vector<double> &w, std::vector<long double> *xl = nullptr) {
   const int Np = p + 1, N = p;
   x.assign(Np, 0.0);
   w.assign(Np, 0.0);
+  if (xl) xl->assign(Np, 0.5L);
   for (int i = 0; i <= N / 2; ++i) {
     long double z = -cosl(3.14159265358979323846264338327950288L * i / N);
     auto legendre = [&](long double zz, long double &PN, long double &PN1) {
@@ -132,6 +133,10 @@ static void gll01(int p, std::vector<double> &x, std::vector<double> &w) {
     legendre(z, PN, PN1);
     const long double wt = 2.0L / (N * (N + 1) * PN * PN);
     x[i] = (double)((1.0L + z) / 2.0L);
+    if (xl) {
+      (*xl)[i] = 2 * i == N ? 0.5L : (1.0L + z) / 2.0L;
+      (*xl)[N - i] = 2 * i == N ? 0.5L : (1.0L - z) / 2.0L;
+    }
     w[i] = (double)(wt / 2.0L);
     x[N - i] = 1.0 - x[i];
     w[N - i] = w[i];
@@ -172,14 +177,35 @@ static void derivative_ops(int p, const std::vector<double> &x, const std::vecto
     b.w[i] = w[i];
     b.iw[i] = 1.0 / w[i];
   }
-  // The two-point fluxes of a line's end node sum to the flux times the
-  // off-diagonal sum of its row, +-1/w0 up to the rounding of the entries (3 to
-  // 4 units at p = 3 and 4); the face flux they nearly cancel with takes the same sum.
-  long double first = 0, last = 0;
-  for (int k = 1; k < Np; ++k) first += b.Dhat2[k];
-  for (int k = 0; k < Np - 1; ++k) last -= b.Dhat2[(Np - 1) * Np + k];
-  b.lift[0] = (double)first;
-  b.lift[1] = (double)last;
+}
+
+// The line form's operator: the off-diagonal entries of 2D from the nodes in
+// long double, each rounded once, antisymmetric (D(p-i, p-l) = -D(i, l)), and the
+// face weight 1/w0 as the sum of an end row.  The two-point fluxes of a line's
+// end node nearly cancel with its face flux, so what the rounding of the row and
+// of the weight leave between them, times the pressure, is most of the error of a
+// low-Mach evaluation: 3 to 4 units of 2^-53 with derivative_ops' entries and
+// 1/w0.  One weight for both ends keeps a face's two sides equal and opposite, and
+// the antisymmetry makes the rows' remainders cancel over an element, so that
+// mass, momentum and energy are conserved to rounding.
+static void line_ops(int p, const std::vector<long double> &x, BasisArgs &b) {
+  const int Np = p + 1;
+  std::vector<long double> wB(Np, 1.0L);
+  for (int i = 0; i < Np; ++i) {
+    for (int j = 0; j < Np; ++j)
+      if (j != i) wB[i] *= x[i] - x[j];
+    wB[i] = 1.0L / wB[i];
+  }
+  for (int i = 0; i <= p / 2; ++i)
+    for (int l = 0; l < Np; ++l) {
+      if (l == i || (2 * i == p && l > i)) continue;  // the middle row's second half by antisymmetry
+      const double d = (double)(2.0L * wB[l] / wB[i] / (x[i] - x[l]));
+      b.D2line[i * Np + l] = d;
+      b.D2line[(p - i) * Np + p - l] = -d;
+    }
+  long double sum = 0;
+  for (int l = 1; l < Np; ++l) sum += b.D2line[l];
+  b.lift = (double)sum;
 }
 
 // Inverse of the 1-D Legendre Vandermonde V(i,a) = P_a(2 x_i - 1) on the
@@ -1082,8 +1108,10 @@ static int create_impl(const theseus_case_desc *desc, const theseus_lte_table *l
   h->Ntot = (long long)ne * h->ndof;
   h->has_boundary = has_boundary;
   std::vector<double> x, w;
-  gll01(d.order, x, w);
+  std::vector<long double> xl;
+  gll01(d.order, x, w, &xl);
   derivative_ops(d.order, x, w, h->basis);
+  line_ops(d.order, xl, h->basis);
   legendre_vandermonde_inverse(d.order, x, h->basis.Vinv);
   init_gas(d, h->gas, h->gas32);
   h->pm = d.precision == THESEUS_PRECISION_MIXED ? 1 : 0;

@@ -54,7 +54,8 @@ struct BasisArgs {
   double Dhat2[MAXNP * MAXNP];  // 2D with the same corner corrections
   double w[MAXNP];              // GLL weights on [0,1]
   double iw[MAXNP];             // their reciprocals
-  double lift[2];               // the line form's face weights at a line's two ends: 1/w0 as Dhat2 has it
+  double D2line[MAXNP * MAXNP];  // the line form's (line_ops): off-diagonal entries of Dhat2,
+  double lift;                   // and 1/w0 as the sum of an end row
   double Vinv[MAXNP * MAXNP];   // inverse 1-D Legendre Vandermonde: mode a = sum_i Vinv[a*Np+i] u_i
 };
 

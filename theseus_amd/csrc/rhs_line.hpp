@@ -483,7 +483,7 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) k_
     for (int c = 0; c < NQ; ++c) rate[m][c] = 0.0;
   double D2[Np * Np];
 #pragma unroll
-  for (int k = 0; k < Np * Np; ++k) D2[k] = B.Dhat2[k];
+  for (int k = 0; k < Np * Np; ++k) D2[k] = B.D2line[k];
 
   double xb[Np][NQ], vd[Np][VISC ? DIM + 1 : 1];
   // unrolled: in a rolled loop the constants of the branches rarely taken
@@ -583,7 +583,7 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) k_
       const int nbe = side ? nhi : nlo;
       const bool bdr = BND && nbe < 0;
       const bool out = side || bdr;  // n points out of the element
-      const double lift = B.lift[side];
+      const double lift = B.lift;
       double n[DIM];
 #pragma unroll
       for (int dd = 0; dd < DIM; ++dd) n[dd] = side ? met[dd] : (bdr ? -met[dd] : nl[dd]);
