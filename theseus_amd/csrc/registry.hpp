@@ -135,12 +135,16 @@ void launch_measures(const MeasArgs &a, int nb, hipStream_t s) {
 //       NS          0.71/0.77  0.87/0.98  0.79/0.87  0.86/0.93  0.86/0.90  1.06/1.07, at 8192 1.03/1.07
 //     Ranocha       0.99/0.85  1.39/1.17  1.02/0.95  1.25/1.06  1.26/1.02  1.61/1.29
 //       boundary    0.94/0.84  1.30/1.13  0.98/0.93  1.20/1.02  1.21/0.98  1.54/1.23
+//     central/Roe   1.25/1.19  1.29/1.28  1.13/1.06  1.35/1.24  1.31/1.14  1.49/1.35, at 512 1.01/0.95
+//     central/LLF   1.44/1.35  1.48/1.42  1.39/1.29  1.65/1.45  1.57/1.37  1.78/1.57, at 512 1.21/1.10
+//       NS          1.23/1.21  1.22/1.24  1.19/1.13  1.27/1.22  1.20/1.18  1.30/1.31, at 512 1.08/1.04
 //   3-D p = 4 (two elements in 50 of 64 lanes, five nodes a lane)
 //     Ranocha/LLF   1.06/0.88  1.08/0.90  0.93/0.93  1.10/1.03  1.14/1.10  1.37/1.15
 //       NS          0.76/0.75  0.95/0.87  0.90/0.91  1.00/0.96  1.00/0.95  1.15/1.05
 //     central/HLL   0.96/0.93  0.93/0.93  0.88/0.91  1.01/0.99  0.96/0.96  1.11/1.05, at 2048 1.18/1.19
 //     Ranocha NS    0.62/0.60  0.95/0.89  0.82/0.83  0.88/0.90  0.90/0.89  1.09/0.97
 //     central/LLF NS 0.81/0.79 0.90/0.93  0.91/0.91  0.99/0.95  0.86/0.87  1.00/1.01, at 8192 0.88/0.93: not built
+// (every pair was measured so, also at 2048, 3072 and 6144 to 27648 waves).
 // The minimum is where both stay above 0.95, the runs' own spread, from there on;
 // without blending the first alone, which in 2-D is lower.  Left out as well, from
 // ratios at 512, 1024, 2048 and 4096 waves without shocks: 3-D p = 4 central/HLL NS
